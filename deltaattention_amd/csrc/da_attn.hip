@@ -1345,33 +1345,82 @@ __global__ __launch_bounds__(kSchedThreads) void hybrid_schedule_kernel(const in
 // fp32 tensors.  The reference's kernels take fp32 Q, K, V as they take 16-bit ones
 // (dtype-agnostic loads, deltaFlashAttention.py:41-42, 80; flashAttention.py:94-130), and
 // p.to(v.dtype) then leaves p in fp32 (:98, :137).  attn_f32_kernel computes the same
-// attention in fp32 throughout: one workgroup of 256 threads per (batch, query head,
-// 64 query rows), LDS tiles of 64 keys, fp32 FMAs on the VALU (the MFMA path is 16-bit),
-// an exact running maximum (rescaled at every new maximum) and P.V on the fp32 p.  The
-// logical 128-row schedule, the key biases log2(w)/c and the variants come from the same
-// schedule pre-pass as the 16-bit kernels.  Thread (ti, tj) holds scores of rows
-// 4 ti .. 4 ti + 3 and keys tj + 16 jj, and output dims 4 tj + 64 gg of the same rows.
+// attention in fp32 throughout on the fp32 matrix instruction v_mfma_f32_32x32x2 (256
+// flops per CU and clock, twice the VALU's unpacked FMA rate, and one operand dword per
+// lane for 4096 flops where the VALU form needs an LDS read per four FMAs): 32 queries a
+// wave, tiles of 32 keys, an exact running maximum (O rescaled at every new maximum) and
+// P.V on the fp32 p.  The logical 128-row schedule, the key biases log2(w)/c and the
+// variants come from the same schedule pre-pass as the 16-bit kernels.
+//
+// Layout.  S^T = K Q^T: a lane holds query ql = lane % 32 and, in register r, key
+// 8 (r / 4) + 4 hl + r % 4 (hl = lane / 32).  O^T += V^T P^T takes the two halves' keys of
+// register r as its two-deep inner dimension, so p[r] is the B operand as it is.  Row i of
+// output block db is head dimension DB i + db, so one load of DB floats of a value row
+// gives a lane its A operands of all DB blocks.  K, Q and V pair the inner dimension as
+// the wide loads bring it (dims 8 m + 4 hl + e).
+//
+// Operands go from L2 to registers, with no LDS: a tile is a stream of fragments (DB of
+// K, NV of V, at most 16 registers each) in a ring of R, loaded R - 1 fragments ahead of
+// their MFMAs (16 MFMAs of 64 cycles each).  Two waves a SIMD cover each other's softmax.
+//
+// A workgroup's four waves split the keys of the same 32 queries: tile t goes to wave
+// t % 4, and the waves' (maximum, sum, O) are merged through LDS at the end.  Whole rows a wave
+// (128 rows a workgroup, the tiles shared through the CU's cache) were slower at every
+// size: 62 against 89 TFLOP/s at 4096 tokens x 32 heads.
+//
+// Measured, dense causal, 128 dims unless said: 2048 tokens x 8 heads of 64 dims 63 us
+// (420 us with the VALU kernel before this one), 1024 x 32 heads 148 (513), 4096 x 32
+// 1557 (6415), 8192 x 32 5.87 ms (20.7; 94 TFLOP/s of 157, the rest is operand loads from
+// L2 and the last-level cache).  Error against 64 bits: 3.0e-7 to 4.6e-7 (before: 4.2e-7
+// to 7.0e-7).  Eight waves a workgroup were 5% faster on grids below two a CU without the
+// pairing below and up to 15% slower elsewhere; a rule between the two would give a ragged
+// batch other sums than its sequences alone.
 // ====================================================================================
-constexpr int kFRows = 64, kFKeys = 64;
-constexpr int kFStride = kD + 4;        // row stride (floats) of the Q, K and V tiles
-constexpr int kFPStride = kFKeys + 4;   // row stride of the P tile
-constexpr int kFLds = (kFRows * kFStride + 2 * kFKeys * kFStride + kFRows * kFPStride + 2 * kFKeys) * 4;
+constexpr int kFRows = 32, kFTile = 32, kFWaves = 4;
 
-template <int VARIANT>
-__global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float fsm[];
-  float* const sQ = fsm;
-  float* const sK = sQ + kFRows * kFStride;
-  float* const sV = sK + kFKeys * kFStride;
-  float* const sP = sV + kFKeys * kFStride;
-  float* const sB = sP + kFRows * kFPStride;  // the tile's key biases (units of the score)
-  int* const sT = (int*)(sB + kFKeys);        // the tile's timestamps (pure Phase 1)
-  const int tid = threadIdx.x;
-  const int ti = tid >> 4, tj = tid & 15;
+template <int VARIANT, int DB>
+struct F32Frags {
+  static constexpr int NV = DB <= 2 ? DB : 4;      // value fragments of a tile
+  static constexpr int NR = 16 / NV;               // S^T registers (key pairs) a value fragment serves
+  static constexpr int F = DB + NV;                // fragments of a tile
+  // ring size; F % R == 0 keeps its slots static (pure Phase 1 at 128 dims has registers for two)
+  static constexpr int R = VARIANT == kPure && DB == 4 ? 2 : F % 4 == 0 ? 4 : F;
+};
+
+template <int VARIANT, int DB>
+__global__ __launch_bounds__(64 * kFWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void attn_f32_kernel(AttnArgs a, int paired) {
+  constexpr int NW = kFWaves;
+  using FR = F32Frags<VARIANT, DB>;
+  __shared__ float s_o[NW * 16 * DB * 64];  // the waves' O, [wave][r][db][lane]
+  __shared__ float s_ml[NW][2][64];         // and their maxima and sums
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, ql = lane & 31;
+  // ---- workgroup -> (head, row block): whole heads per XCD where they split evenly, the
+  // longest row blocks first.  A grid of at most two workgroups a CU (paired) starts all at
+  // once, each CU taking one of the first half and one of the second: there the second half
+  // runs from the shortest up, so that every CU gets about the same work (2048 tokens x 8
+  // heads of 64 dims: 63 us, 80 with the longest first throughout) ----
   const int nrb = (a.Nq + kFRows - 1) / kFRows;
-  const int rb = (int)(blockIdx.x % (unsigned)nrb);
-  const int bh = (int)(blockIdx.x / (unsigned)nrb);
-  const int h = bh % a.Hq, b = bh / a.Hq;
+  const int units = a.B * a.Hq;
+  int unit, rb;
+  if (paired) {
+    const int nx = (units & 7) == 0 ? 8 : 1;
+    const int upx = units / nx, n = upx * nrb;  // an XCD's heads and workgroups
+    const int idx = blockIdx.x / nx, half = (n + 1) >> 1;
+    const int e = idx < half ? idx : n - 1 - (idx - half);
+    unit = (int)(blockIdx.x % nx) * upx + e % upx;
+    rb = nrb - 1 - e / upx;
+  } else if ((units & 7) == 0) {
+    const int idx = blockIdx.x >> 3;
+    unit = (blockIdx.x & 7) * (units >> 3) + idx / nrb;
+    rb = nrb - 1 - idx % nrb;
+  } else {
+    unit = blockIdx.x % units;
+    rb = nrb - 1 - blockIdx.x / units;
+  }
+  const int h = unit % a.Hq, b = unit / a.Hq;
   const int g = h / a.G;
   const int bg = b * a.Hkv + g;
   const int Nq = a.seq.cu ? a.seq.len(b) : a.Nq;
@@ -1394,15 +1443,16 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
     const int nblk = (P + kBlock - 1) / kBlock;
     const int32_t* bmax = a.sched + (int64_t)bg * 2 * a.nblk_cap;
     int n_safe, last;
-    safe_prefix(bmax, bmax + a.nblk_cap, nblk, start_m - a.window, n_safe, last, tid & 63);
+    safe_prefix(bmax, bmax + a.nblk_cap, nblk, start_m - a.window, n_safe, last, lane);
     ds = max(0, ((last + 1) / kBlock) * kBlock);
     if (VARIANT == kHybrid) n1 = min(n_safe * kBlock, a.wcap);
   } else if (VARIANT == kPure) {
     n1 = P;
     kend = 0;
   }
-  const int t1 = (n1 + kFKeys - 1) / kFKeys;
-  const int t2 = kend > ds ? (kend - ds + kFKeys - 1) / kFKeys : 0;
+  const int t1 = (n1 + kFTile - 1) / kFTile;
+  const int t2 = kend > ds ? (kend - ds + kFTile - 1) / kFTile : 0;
+  const int T = t1 + t2;
 
   const float* qg = (const float*)a.q + a.seq.base(b, a.sq_b, a.sq_n) + (int64_t)h * a.sq_h;
   const float* kg = (const float*)a.k + a.seq.base(b, a.sk_b, a.sk_n) + (int64_t)g * a.sk_h;
@@ -1412,150 +1462,163 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnArgs a) {
   const float* wrow = a.wts ? a.wts + (int64_t)bg * a.wcap : nullptr;
   const int32_t* tsrow = a.tsw ? a.tsw + (int64_t)bg * a.wcap : nullptr;
 
-  // ---- Q of the 64 rows (rows past Nq and dims past D are zero) ----
-  for (int i = tid; i < kFRows * (kD / 4); i += 256) {
-    const int r = i / (kD / 4), d = 4 * (i % (kD / 4));
-    float4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (R0 + r < Nq && d < D) x = *(const float4*)(qg + (int64_t)(R0 + r) * a.sq_n + d);
-    *(float4*)(sQ + r * kFStride + d) = x;
+  // ---- Q^T: dims 8 m + 4 hl .. + 3 of query R0 + ql (rows past Nq and dims past D zero) ----
+  const int row = R0 + ql;
+  f32x4 qf[4 * DB];
+#pragma unroll
+  for (int m = 0; m < 4 * DB; ++m) {
+    const bool in = row < Nq && 8 * m < D;
+    qf[m] = in ? *(const f32x4*)(qg + (int64_t)row * a.sq_n + 8 * m + 4 * hl) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
 
-  float o[4][2][4];
-  float m[4], l[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.0f;
-#pragma unroll
-    for (int gg = 0; gg < 2; ++gg)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[i][gg][e] = 0.0f;
-  }
-
-  for (int t = 0; t < t1 + t2; ++t) {
+  // Fragment f of tile t.  Keys past the source's end repeat its last row (a row of the
+  // same tile) and get no weight; dims past D are zero (K) or never stored (V).  A row is a
+  // scalar tile base plus a 32-bit lane offset (below 32 rows of less than 2^25 bytes).
+  auto load = [&](auto FC, const int t, float (&x)[16]) {
+    constexpr int f = decltype(FC)::value;
     const bool ph1 = t < t1;
-    const int key0 = ph1 ? t * kFKeys : ds + (t - t1) * kFKeys;
-    if (!ph1 && a.causal && key0 > R0 + kFRows - 1) break;  // every later tile is masked
-    const int kvalid = ph1 ? n1 : kend;  // keys [key0, kvalid) of this tile are real
-    const int klimit = ph1 ? P : Nk;     // rows of the source tensor that exist
-    const float* ksrc = ph1 ? kpg : kg;
-    const float* vsrc = ph1 ? vpg : vg;
-    const int64_t skn = ph1 ? a.skp_n : a.sk_n, svn = ph1 ? a.svp_n : a.sv_n;
-    __syncthreads();  // the previous tile's K, V, P and biases are read
-    for (int i = tid; i < kFKeys * (kD / 4); i += 256) {
-      const int r = i / (kD / 4), d = 4 * (i % (kD / 4));
-      const int key = key0 + r;
-      float4 kx = {0.0f, 0.0f, 0.0f, 0.0f}, vx = kx;
-      if (key < kvalid && key < klimit && d < D) {
-        kx = *(const float4*)(ksrc + (int64_t)key * skn + d);
-        vx = *(const float4*)(vsrc + (int64_t)key * svn + d);
+    const int key0 = ph1 ? t * kFTile : ds + (t - t1) * kFTile;
+    const unsigned last = (unsigned)((ph1 ? P : Nk) - 1 - key0);
+    const unsigned sn = (unsigned)(f < DB ? (ph1 ? a.skp_n : a.sk_n) : (ph1 ? a.svp_n : a.sv_n));
+    const float* base = (f < DB ? (ph1 ? kpg : kg) : (ph1 ? vpg : vg)) + (int64_t)key0 * sn;
+    // opaque: the rows' offsets are formed here, not held in registers across tiles
+    int ql = lane & 31, hl = lane >> 5;
+    asm volatile("" : "+v"(ql), "+v"(hl));
+    if constexpr (f < DB) {
+      const unsigned off = min((unsigned)ql, last) * sn + 4 * hl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int m = 4 * f + u;
+        const f32x4 w = 8 * m < D ? *(const f32x4*)(base + off + 8 * m) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * u + e] = w[e];
       }
-      *(float4*)(sK + r * kFStride + d) = kx;
-      *(float4*)(sV + r * kFStride + d) = vx;
-    }
-    if (tid < kFKeys) {
-      const int key = key0 + tid;
-      float bias = key < kvalid ? 0.0f : -INFINITY;
-      int ts = 0;
-      if (ph1 && (VARIANT == kHybrid || VARIANT == kPure) && key < kvalid) bias = wrow[key];
-      if (ph1 && VARIANT == kPure && key < kvalid) ts = tsrow[key];
-      sB[tid] = bias;
-      sT[tid] = ts;
-    }
-    __syncthreads();
-
-    // ---- scores of rows 4 ti + i and keys tj + 16 jj ----
-    float sc[4][4];
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int u = 0; u < FR::NR; ++u) {
+        const int r = (f - DB) * FR::NR + u;
+        const unsigned off = min((unsigned)(8 * (r >> 2) + 4 * hl + (r & 3)), last) * sn;
+        struct __attribute__((packed, aligned(4))) Row { float v[DB]; };
+        if (D == 32 * DB) {
+          const Row w = *(const Row*)(base + off + DB * ql);
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) sc[i][jj] = 0.0f;
-    for (int d = 0; d < D; d += 4) {
-      float4 qv[4], kv[4];
+          for (int e = 0; e < DB; ++e) x[DB * u + e] = w.v[e];
+        } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) qv[i] = *(const float4*)(sQ + (4 * ti + i) * kFStride + d);
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) kv[jj] = *(const float4*)(sK + (tj + 16 * jj) * kFStride + d);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          sc[i][jj] = __builtin_fmaf(qv[i].x, kv[jj].x, sc[i][jj]);
-          sc[i][jj] = __builtin_fmaf(qv[i].y, kv[jj].y, sc[i][jj]);
-          sc[i][jj] = __builtin_fmaf(qv[i].z, kv[jj].z, sc[i][jj]);
-          sc[i][jj] = __builtin_fmaf(qv[i].w, kv[jj].w, sc[i][jj]);
-        }
-    }
-    // ---- masks, online softmax (exact maximum), p to LDS ----
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = R0 + 4 * ti + i;
-      float mt = -INFINITY;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int kl = tj + 16 * jj;
-        bool ok = sB[kl] != -INFINITY;
-        if (!ph1 && a.causal) ok = ok && key0 + kl <= row;                 // deltaFlashAttention.py:126-130
-        if (VARIANT == kPure) ok = ok && sT[kl] <= row;                    // :338-341
-        sc[i][jj] = ok ? (sc[i][jj] + sB[kl]) * c : -INFINITY;
-        mt = __builtin_fmaxf(mt, sc[i][jj]);
-      }
-#pragma unroll
-      for (int x = 1; x < 16; x <<= 1) mt = __builtin_fmaxf(mt, __shfl_xor(mt, x, 64));
-      const float mn = __builtin_fmaxf(m[i], mt);
-      const float alpha = mn == -INFINITY ? 1.0f : exp2f(m[i] - mn);
-      float ps = 0.0f;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const float pv = mn == -INFINITY ? 0.0f : exp2f(sc[i][jj] - mn);
-        ps += pv;
-        sP[(4 * ti + i) * kFPStride + tj + 16 * jj] = pv;
-      }
-#pragma unroll
-      for (int x = 1; x < 16; x <<= 1) ps += __shfl_xor(ps, x, 64);
-      l[i] = l[i] * alpha + ps;
-      m[i] = mn;
-#pragma unroll
-      for (int gg = 0; gg < 2; ++gg)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[i][gg][e] *= alpha;
-    }
-    __syncthreads();
-    // ---- O += P V on dims 4 tj + 64 gg ----
-    for (int j = 0; j < kFKeys; ++j) {
-      float pj[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) pj[i] = sP[(4 * ti + i) * kFPStride + j];
-#pragma unroll
-      for (int gg = 0; gg < 2; ++gg) {
-        const float4 vv = *(const float4*)(sV + j * kFStride + 4 * tj + 64 * gg);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          o[i][gg][0] = __builtin_fmaf(pj[i], vv.x, o[i][gg][0]);
-          o[i][gg][1] = __builtin_fmaf(pj[i], vv.y, o[i][gg][1]);
-          o[i][gg][2] = __builtin_fmaf(pj[i], vv.z, o[i][gg][2]);
-          o[i][gg][3] = __builtin_fmaf(pj[i], vv.w, o[i][gg][3]);
+          for (int e = 0; e < DB; ++e) x[DB * u + e] = base[off + min(DB * ql + e, D - 1)];
         }
       }
     }
+  };
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o[db] = f32x16{};
+  float m_i = -INFINITY, l_i = 0.0f;
+  float ring[FR::R][16];
+
+  int t = wid;
+  if (t < T)
+    static_for<FR::R - 1>([&](auto FC) { load(FC, t, ring[decltype(FC)::value]); });
+  for (; t < T; t += NW) {
+    const bool ph1 = t < t1;
+    const int key0 = ph1 ? t * kFTile : ds + (t - t1) * kFTile;
+    const int tn = min(t + NW, T - 1);  // past the last tile: loaded again, never used
+    // fragment f + R - 1 goes out before fragment f is used
+    auto ahead = [&](auto FC) {
+      constexpr int n = decltype(FC)::value + FR::R - 1;
+      load(std::integral_constant<int, n % FR::F>{}, n < FR::F ? t : tn, ring[n % FR::R]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    f32x16 s = f32x16{};
+    static_for<DB>([&](auto FC) {
+      constexpr int f = decltype(FC)::value;
+      ahead(FC);
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(ring[f % FR::R][u], qf[4 * f + (u >> 2)][u & 3], s, 0, 0, 0);
+    });
+    // ---- masks, online softmax (exact maximum) ----
+    float mt = -INFINITY;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const int kl = key0 + 8 * r4 + 4 * hl;
+      f32x4 bias = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      int4 ts = {0, 0, 0, 0};
+      if ((VARIANT == kHybrid || VARIANT == kPure) && ph1) bias = *(const f32x4*)(wrow + kl);
+      if (VARIANT == kPure) ts = *(const int4*)(tsrow + kl);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        bool ok = bias[e] != -INFINITY;
+        if (!ph1) ok = ok && kl + e < kend && (!a.causal || kl + e <= row);     // deltaFlashAttention.py:126-130
+        if (VARIANT == kPure) ok = ok && (e == 0 ? ts.x : e == 1 ? ts.y : e == 2 ? ts.z : ts.w) <= row;  // :338-341
+        s[4 * r4 + e] = ok ? (s[4 * r4 + e] + bias[e]) * c : -INFINITY;
+        mt = __builtin_fmaxf(mt, s[4 * r4 + e]);
+      }
+    }
+    const float mn = __builtin_fmaxf(m_i, halves_max(mt));
+    const float alpha = mn == -INFINITY ? 1.0f : exp2f(m_i - mn);
+    float ps = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = mn == -INFINITY ? 0.0f : exp2f(s[r] - mn);
+      ps += s[r];
+    }
+    l_i = l_i * alpha + ps;
+    m_i = mn;
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+    }
+    // ---- O^T += V^T P^T ----
+    static_for<FR::NV>([&](auto VC) {
+      constexpr int fv = decltype(VC)::value;
+      ahead(std::integral_constant<int, DB + fv>{});
+#pragma unroll
+      for (int u = 0; u < FR::NR; ++u)
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(ring[(DB + fv) % FR::R][DB * u + db], s[fv * FR::NR + u],
+                                                       o[db], 0, 0, 0);
+    });
   }
 
-  // ---- normalise and store rows < Nq, dims < D ----
-  float* og = (float*)a.out + a.seq.base(b, a.so_b, a.so_n) + (int64_t)h * a.so_h;
+  // ---- merge: wave w adds up registers kOwn w .. + kOwn - 1 (kOwn DB consecutive dims
+  // of the lane's row) of all waves, normalises and stores rows < Nq, dims < D ----
+  constexpr int kOwn = 16 / NW;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = R0 + 4 * ti + i;
-    if (row >= Nq) continue;
-    // a row without any key (pure Phase 1) stays zero, deltaFlashAttention.py:353-354
-    const float inv = l[i] > 0.0f ? 1.0f / l[i] : 0.0f;
+  for (int r = 0; r < 16; ++r)
 #pragma unroll
-    for (int gg = 0; gg < 2; ++gg) {
-      const int d = 4 * tj + 64 * gg;
-      if (d < D)
-        *(float4*)(og + (int64_t)row * a.so_n + d) =
-            float4{o[i][gg][0] * inv, o[i][gg][1] * inv, o[i][gg][2] * inv, o[i][gg][3] * inv};
-    }
+    for (int db = 0; db < DB; ++db) s_o[((wid * 16 + r) * DB + db) * 64 + lane] = o[db][r];
+  s_ml[wid][0][lane] = m_i;
+  s_ml[wid][1][lane] = halves_sum(l_i);
+  __syncthreads();
+  float M = -INFINITY, L = 0.0f, f[NW];
+#pragma unroll
+  for (int w = 0; w < NW; ++w) M = __builtin_fmaxf(M, s_ml[w][0][lane]);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    f[w] = M == -INFINITY ? 0.0f : exp2f(s_ml[w][0][lane] - M);
+    L += s_ml[w][1][lane] * f[w];
   }
+  // a row without any key (pure Phase 1) stays zero, deltaFlashAttention.py:353-354
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  float x[kOwn * DB];
+#pragma unroll
+  for (int i = 0; i < kOwn * DB; ++i) {
+    x[i] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) x[i] += s_o[((w * 16 + kOwn * wid) * DB + i) * 64 + lane] * f[w];
+    x[i] *= inv;
+  }
+  if (row >= Nq) return;
+  const int r0 = kOwn * wid, d0 = DB * (8 * (r0 >> 2) + 4 * hl + (r0 & 3));
+  float* orow = (float*)a.out + a.seq.base(b, a.so_b, a.so_n) + (int64_t)h * a.so_h + (int64_t)row * a.so_n;
+#pragma unroll
+  for (int i = 0; i < kOwn * DB; i += 2)  // D is even: two dims are both in or both out
+    if (d0 + i < D) *(f32x2*)(orow + d0 + i) = f32x2{x[i], x[i + 1]};
 }
 
 template <int V, int DT>
@@ -1635,28 +1698,32 @@ static int launch_attn_dt(int variant, AttnArgs& a, hipStream_t st) {
   }
 }
 
-template <int V>
+template <int V, int DB>
 static int launch_attn_f32_t(const AttnArgs& a, hipStream_t st) {
-  static int done = 0;
-  if (!done) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<V>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kFLds);
-    if (e != hipSuccess) return set_error(DA_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-    done = 1;
-  }
   const int64_t grid = (int64_t)a.B * a.Hq * ((a.Nq + kFRows - 1) / kFRows);
   if (grid >= (1ll << 31)) return set_error(DA_ERR_INVALID, "attention (fp32): grid too large");
-  hipLaunchKernelGGL((attn_f32_kernel<V>), dim3((unsigned)grid), dim3(256), kFLds, st, a);
+  hipLaunchKernelGGL((attn_f32_kernel<V, DB>), dim3((unsigned)grid), dim3(64 * kFWaves), 0, st, a,
+                     grid <= 2 * cu_count() ? 1 : 0);
   return check_launch("attention kernel (fp32)");
+}
+
+template <int V>
+static int launch_attn_f32(const AttnArgs& a, hipStream_t st) {
+  switch ((a.D + 31) / 32) {
+    case 1: return launch_attn_f32_t<V, 1>(a, st);
+    case 2: return launch_attn_f32_t<V, 2>(a, st);
+    case 3: return launch_attn_f32_t<V, 3>(a, st);
+    default: return launch_attn_f32_t<V, 4>(a, st);
+  }
 }
 
 static int launch_attn(int variant, int dtype, AttnArgs& a, hipStream_t st) {
   if (dtype == DA_F32) {
     switch (variant) {
-      case kHybrid: return launch_attn_f32_t<kHybrid>(a, st);
-      case kSanity: return launch_attn_f32_t<kSanity>(a, st);
-      case kPure: return launch_attn_f32_t<kPure>(a, st);
-      default: return launch_attn_f32_t<kDense>(a, st);
+      case kHybrid: return launch_attn_f32<kHybrid>(a, st);
+      case kSanity: return launch_attn_f32<kSanity>(a, st);
+      case kPure: return launch_attn_f32<kPure>(a, st);
+      default: return launch_attn_f32<kDense>(a, st);
     }
   }
   return dtype == DA_F16 ? launch_attn_dt<DA_F16>(variant, a, st) : launch_attn_dt<DA_BF16>(variant, a, st);
