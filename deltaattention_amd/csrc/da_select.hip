@@ -25,10 +25,11 @@
 // scalar round trip), the anchor update is a select, and a batch's decisions collect
 // in a 32-bit mask stored as int32 (the reference's keep-mask format).
 //
-// From 2048 chunks on (two per SIMD), select_pair_kernel walks two chunks per wave,
-// one per 32-lane half with four slots per lane, over the same tree (bit-identical);
-// below that, one wave per chunk keeps every chunk on a SIMD of its own.
+// That walk is select_kernel.  Rows a matrix operand can be loaded from take
+// select_band_kernel instead, which decides most (anchor, row) pairs of a chunk from
+// matrix products, all at once, and leaves only the close ones to the exact tree.
 #include <algorithm>
+#include <cmath>
 
 #include "da_common.hpp"
 
@@ -36,6 +37,7 @@ namespace da {
 
 constexpr int kSelBatch = 32;
 constexpr int64_t kSelPairMinChunks = 2048;
+constexpr int64_t kBandMinRows = 96;
 
 // x rounded to the 16-bit type DT (nearest even) and widened back to fp32.  For bf16
 // one v_cvt_pk_bf16_f32 with x in the high half and 0 in the low half leaves exactly
@@ -183,16 +185,19 @@ __global__ __launch_bounds__(256) void select_kernel(
   if (lane == 0) chunk_counts[w] = count;  // tritonModules.py:68-69
 }
 
-// ---- two chunks per wave, one per 32-lane half ----
-// Lane q of a half holds head-dimension slots 4q .. 4q+3 of a row (one 8-byte load), so
-// a wave walks two chunks at once.  The tree keeps its pairing: levels 1-2 add slots
+// ---- two pairs per wave, one per 32-lane half ----
+// Lane q of a half holds head-dimension slots 4q .. 4q+3 of a row, so a wave decides two
+// pairs in one instruction stream.  The tree keeps its pairing: levels 1-2 add slots
 // inside the lane, lane^1, lane^2, the 8-lane and the 16-lane mirror give levels 3-6, and
 // v_permlane16_swap pairs the two 16-lane rows of each half for level 7 -- the blocks
-// that the one-chunk-per-wave tree pairs at each level, so the sums are bit-identical.
+// that the one-row-per-wave tree pairs at each level, so the sums are bit-identical.
 template <bool R16, int DT>
 __device__ __forceinline__ float half_tree_sum(float p0, float p1, float p2, float p3) {
 #pragma clang fp contract(off)
-  auto r = [](float v) { return R16 ? round16<DT>(v) : v; };
+  auto r = [](float v) {
+    if constexpr (R16) return round16<DT>(v);
+    else return v;
+  };
   float t = r(r(p0 + p1) + r(p2 + p3));
   t = r(t + dpp_f32<kDppXor1>(t));
   t = r(t + dpp_f32<kDppXor2>(t));
@@ -202,6 +207,53 @@ __device__ __forceinline__ float half_tree_sum(float p0, float p1, float p2, flo
   return r(__uint_as_float(sw[0]) + __uint_as_float(sw[1]));
 }
 
+// Four slots of a row.
+template <int DT>
+struct HalfKey {
+  using Row = u32x2;
+  static __device__ __forceinline__ float at(Row w, int i) {
+    return i & 1 ? E16<DT>::hi(w[i >> 1]) : E16<DT>::lo(w[i >> 1]);
+  }
+};
+template <>
+struct HalfKey<DA_F32> {
+  using Row = f32x4;
+  static __device__ __forceinline__ float at(Row w, int i) { return w[i]; }
+};
+
+// select_step's decision for the row (x) and the anchor (a) a 32-lane half holds.
+template <bool COS, bool A16, int DT>
+__device__ __forceinline__ bool half_keep(typename HalfKey<DT>::Row xb, typename HalfKey<DT>::Row ab, float thr) {
+#pragma clang fp contract(off)
+  float x[4], a[4], p[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = HalfKey<DT>::at(xb, i);
+    a[i] = HalfKey<DT>::at(ab, i);
+  }
+  if constexpr (COS) {  // tritonModules.py:48-54
+    const float dot = half_tree_sum<false, DT>(x[0] * a[0], x[1] * a[1], x[2] * a[2], x[3] * a[3]);
+    const float xn = sqrt_rn(half_tree_sum<false, DT>(x[0] * x[0], x[1] * x[1], x[2] * x[2], x[3] * x[3]) + 1e-8f);
+    const float an = sqrt_rn(half_tree_sum<false, DT>(a[0] * a[0], a[1] * a[1], a[2] * a[2], a[3] * a[3]) + 1e-8f);
+    return __fdiv_rn(dot, xn * an) < thr;
+  } else if constexpr (A16) {  // tritonModules.py:55-58 in the keys' 16-bit arithmetic
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float d = round16<DT>(x[i] - a[i]);
+      p[i] = round16<DT>(d * d);
+    }
+    return half_tree_sum<true, DT>(p[0], p[1], p[2], p[3]) > thr;
+  } else {  // tritonModules.py:55-58
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float d = x[i] - a[i];
+      p[i] = d * d;
+    }
+    return half_tree_sum<false, DT>(p[0], p[1], p[2], p[3]) > thr;
+  }
+}
+
+// ---- two chunks per wave, one per 32-lane half ----
 // select_step for the row a 32-lane half holds (x: four slots); rows with `valid` false
 // are never kept.
 template <bool COS, bool A16, int DT>
@@ -302,6 +354,381 @@ __global__ __launch_bounds__(256) void select_pair_kernel(
   if (q == 0 && e > s) chunk_counts[w] = count;  // tritonModules.py:68-69
 }
 
+// ---- the banded walk ----
+// The chain of the walk above is one exact distance per row (about 30 dependent
+// instructions, 0.14 us), 511 of them in a chunk, whatever the number of chunks.  But which
+// rows are compared with which anchor only matters after the fact: with
+//     next(i) = the first row after i that is kept against anchor i
+// known for every row i, the anchors are 0, next(0), next(next(0)), ...  select_band_kernel
+// finds next(i) for all rows of a chunk at once.  One workgroup of 8 waves takes a chunk in
+// segments of 512 rows, a wave two tiles of 32 anchors each:
+//
+// 1. Gram tiles (v_mfma_f32_32x32x16): the wave's anchors against their own tile and the
+//    next one, i.e. the 32 to 63 rows that follow each anchor.  With the rows' squared norms
+//    (fp32) each pair's distance (or cosine) follows to within a proven bound, and the pair
+//    is kept, dropped or open (three states, two bits, in the anchor's lane).
+// 2. The open pairs that come first in an anchor's row of bits are decided by the exact tree
+//    of the walk, two per wave and four such in one instruction stream, until every anchor's first kept
+//    row is known (about 0.4 pairs an anchor in bf16 arithmetic at one key in four kept,
+//    near none in fp32 arithmetic).
+// 3. Each wave follows the chain inside its 64 rows from all of them at once (pointer
+//    doubling between lanes), one wave joins the eight blocks.  An anchor that keeps none of
+//    the rows its tiles cover (or that 2 did not get to: keys all about as far apart as the
+//    threshold) scans on with the exact tree, eight rows a stream.
+//
+// Every decision is either proven by its bound or the exact tree's, so the result is the
+// walk's bit for bit.  The bounds, with u the unit roundoff of the walk's arithmetic:
+// * Gram: the products of 16-bit elements are exact and the 128 of them (and the norms'
+//   squares) are added in fp32, so |e - d2| <= 2^-15 (n_a + n_c) for e = n_a + n_c - 2 g (128
+//   additions of at most 2^-23 of sum |x y| <= (n_a + n_c) / 2 each, twice, and the norms').
+//   fp32 keys are rounded to bf16 for the products (u = 2^-8 an element): 2^-6.9 instead.
+// * The walk's own distance S rounds the difference (twice in the square), the square and
+//   seven tree levels: d2 (1 - u)^10 <= S <= d2 (1 + u)^10.  In fp16 a square below 2^-14 is
+//   rounded to a multiple of 2^-24: 2^-17 more for 128 of them; sums past 65504 become
+//   infinite, so nothing above 60000 is dropped.
+// * Cosine: |sim - g / sqrt((n_a + 1e-8)(n_c + 1e-8))| <= 2^-14 (2^-6.5 for fp32 keys).
+// * Rows with a norm at or above 2^120 (or infinite, or NaN) leave all their pairs open; a
+//   threshold below 1e-28 drops nothing, and nothing below 1e-30 is kept unseen.
+//
+// Measured, the selection alone, 8 heads of bf16 keys, one in four kept: 1531 keys 17 us
+// (71 with the serial walk), 32768 30 (75), 65536 50 (77, one in two); 8192 keys in one
+// chunk 0.22 ms (1.07).  What is left at few chunks is a chain of loads (the tiles, the
+// exact decisions' rows, five or six streams a wave); at many, reading the keys (75 of 108
+// us at 131072) and the exact decisions (32).
+constexpr int kBandSeg = 512, kBandWaves = 8;
+constexpr int kBandEval = 4;     // exact decisions in one instruction stream, two each
+constexpr int kBandRounds = 24;  // streams a wave spends on its 64 anchors before it leaves the rest to 3
+
+struct BandBounds {
+  float c_lo, c_hi;  // e's lower and upper bound: c (n_a + n_c) - 2 g
+  float keep, drop;  // kept above / dropped below (Euclidean), kept below / dropped above (cosine)
+};
+
+// The bounds of one threshold (host).
+static BandBounds band_bounds(bool cosine, bool a16, int dtype, float thr) {
+  BandBounds b = {};
+  const double t = thr;
+  if (cosine) {
+    const double d = dtype == DA_F32 ? std::ldexp(1.0, -6) * 0.70710678 : std::ldexp(1.0, -14);
+    b.keep = (float)(t - d - 1e-6);
+    b.drop = (float)(t + d + 1e-6);
+    return b;
+  }
+  const double g = dtype == DA_F32 ? 0.0084 : std::ldexp(1.0, -15);
+  const double u = !a16 || dtype == DA_F32 ? std::ldexp(1.0, -24) : std::ldexp(1.0, dtype == DA_BF16 ? -8 : -11);
+  const double tiny = a16 && dtype == DA_F16 ? std::ldexp(1.0, -17) : 0.0;
+  const double slack = 1.0 + std::ldexp(1.0, -18);  // the bounds' own fp32 arithmetic
+  b.c_lo = (float)(1.0 - g);
+  b.c_hi = (float)(1.0 + g);
+  b.keep = (float)std::max((t + tiny) / std::pow(1.0 - u, 10) * (t > 0 ? slack : 1.0), 1e-30);
+  double drop = (t - tiny) / std::pow(1.0 + u, 10) / slack;
+  if (a16 && dtype == DA_F16) drop = std::min(drop, 60000.0);
+  b.drop = t < 1e-28 ? -INFINITY : (float)drop;
+  return b;
+}
+
+// A tile of 32 rows as matrix operands: lane (ql, hl) holds dims 16 t + 8 hl .. + 7 of row
+// ql, and the lane's share of the row's squared norm.
+template <int DT>
+struct BandTile {
+  u32x4 w[8];
+  float n;
+};
+
+// The loads go out together: chunks at or past D repeat the row's last one and are zeroed
+// after (a guarded load would be waited for before the next one).
+template <int DT, bool FULL>
+__device__ __forceinline__ void band_load(BandTile<DT>& x, const typename SelKey<DT>::Elem* row, int D, int hl) {
+  if constexpr (DT == DA_F32) {
+    // converted here: the norm is of the fp32 elements, the products of their bf16 roundings
+    f32x4 lo[8], hi[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int d = FULL ? 16 * t + 8 * hl : min(16 * t + 8 * hl, D - 8);
+      lo[t] = *(const f32x4*)(row + d);
+      hi[t] = *(const f32x4*)(row + d + 4);
+    }
+    x.n = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const bool in = FULL || 16 * t + 8 * hl < D;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lo[t][i] = in ? lo[t][i] : 0.0f;
+        hi[t][i] = in ? hi[t][i] : 0.0f;
+        x.n = __builtin_fmaf(lo[t][i], lo[t][i], __builtin_fmaf(hi[t][i], hi[t][i], x.n));
+      }
+      x.w[t] = u32x4{pack_bf16x2(lo[t][0], lo[t][1]), pack_bf16x2(lo[t][2], lo[t][3]),
+                     pack_bf16x2(hi[t][0], hi[t][1]), pack_bf16x2(hi[t][2], hi[t][3])};
+    }
+  } else {
+    if constexpr (FULL) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) x.w[t] = *(const u32x4*)(row + 8 * hl + 16 * t);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) x.w[t] = *(const u32x4*)(row + min(16 * t + 8 * hl, D - 8));
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x.w[t][i] = 16 * t + 8 * hl < D ? x.w[t][i] : 0u;
+    }
+  }
+}
+
+// Gram tile: lane (ql, hl) gets row ql of b against rows 8 (r / 4) + 4 hl + r % 4 of a.
+template <int DT>
+__device__ __forceinline__ f32x16 band_gram(const BandTile<DT>& a, const BandTile<DT>& b) {
+  f32x16 g = f32x16{};
+#pragma unroll
+  for (int t = 0; t < 8; ++t) g = E16<DT == DA_F16 ? DA_F16 : DA_BF16>::mfma(a.w[t], b.w[t], g);
+  return g;
+}
+
+// The squared norm of row ql, in both halves: the diagonal of the tile's own Gram tile
+// (an eighth of the instructions of unpacking and squaring the row).
+template <int DT>
+__device__ __forceinline__ float band_norm(const BandTile<DT>& x, int ql, int hl) {
+  float n = 0.0f;
+  if constexpr (DT == DA_F32) {
+    n = x.n;
+  } else {
+    const f32x16 g = band_gram<DT>(x, x);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) n = ql - 4 * hl == 8 * (r >> 2) + (r & 3) ? g[r] : n;
+  }
+  return n + swap_halves(n);
+}
+
+// FULL: D = 128 (rows at immediate offsets from one address; two workgroups a CU then fit
+// the registers of the Euclidean walk on 16-bit keys).
+template <bool COS, bool A16, int DT, bool FULL>
+__global__ __launch_bounds__(64 * kBandWaves) __attribute__((amdgpu_waves_per_eu(FULL && !COS && DT != DA_F32 ? 4 : 2)))
+void select_band_kernel(
+    const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int H, int64_t N,
+    int D_arg, int cs, int nc, float thr, BandBounds bounds, int32_t* __restrict__ keep,
+    int32_t* __restrict__ chunk_counts, SeqMap seq, int64_t keep_sh, int divide_to) {
+  __shared__ float s_norm[kBandWaves][2][32];     // a wave's candidates' norms (cosine: 1 / norm)
+  __shared__ u32x2 s_path[kBandSeg];              // the chain from a row, inside its block of 64
+  __shared__ uint8_t s_to[kBandSeg];              // and where it leads
+  __shared__ uint8_t s_from[kBandSeg];
+  __shared__ uint64_t s_bits[kBandSeg / 64];
+  __shared__ int s_cur;
+  const int D = FULL ? 128 : D_arg;
+  const int tid = threadIdx.x;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int lane = tid & 63, ql = lane & 31, hl = lane >> 5;
+  // 32 bits are enough for the chunk's place (the grid, N and the chunks are below 2^31)
+  const unsigned w = blockIdx.x;
+  const unsigned bh = w / (unsigned)nc;
+  const unsigned c = w - bh * (unsigned)nc;
+  const unsigned b = bh / (unsigned)H, h = bh - b * (unsigned)H;
+  const unsigned Nb = seq.cu ? seq.len((int)b) : (int)N;
+  unsigned csb = (unsigned)cs;
+  if (seq.cu) csb = divide_to > 0 ? (Nb + divide_to - 1) / divide_to : min(csb, Nb);
+  const int64_t s64 = (int64_t)c * csb;
+  if (Nb == 0 || s64 >= Nb) {  // tritonModules.py:34-35 (count stays 0, modeling_llama.py:637)
+    if (tid == 0) chunk_counts[w] = 0;
+    return;
+  }
+  const int s = (int)s64;
+  const int e = (int)(s64 + csb < Nb ? s64 + csb : Nb);
+  using Elem = typename SelKey<DT>::Elem;
+  using Row = typename HalfKey<DT>::Row;
+  const Elem* base = (const Elem*)(const void*)k + seq.base((int)b, sk_b, sk_n) + (int64_t)h * sk_h;
+  int32_t* keep_row = keep + (seq.cu ? (int64_t)h * keep_sh + seq.start((int)b) : (int64_t)bh * N);
+  // the exact decisions' operands: a half-wave's row
+  auto row_bits = [&](int r) -> Row {
+    Row x = *(const Row*)(base + (int64_t)r * sk_n + (FULL ? 4 * ql : min(4 * ql, D - 4)));
+    if constexpr (!FULL) {
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(Row) / 4); ++i) x[i] = 4 * ql < D ? x[i] : 0;
+    }
+    return x;
+  };
+  auto load_tile = [&](BandTile<DT>& x, int tb) {  // rows past the chunk repeat its last one
+    band_load<DT, FULL>(x, base + (int64_t)min(tb + ql, e - 1) * sk_n, D, hl);
+  };
+
+  int cur = s;  // the next anchor
+  int count = 0;
+  const int seg = blockDim.x;  // rows a segment: 64 a wave
+  for (int sb = s; sb < e; sb += seg) {
+    // opaque: what derives from the lane is formed here, not held in registers over the loop
+    asm volatile("" : "+v"(lane), "+v"(ql), "+v"(hl));
+    const int se = min(sb + seg, e);
+    if (cur < se) {
+      const int tb = sb + 64 * wid;  // the wave's anchors: tiles tb and tb + 32
+      if (tb < se && tb + 63 >= cur) {
+        BandTile<DT> x, y;
+        load_tile(x, tb);
+        load_tile(y, tb + 32);
+        float nx = band_norm<DT>(x, ql, hl);
+        // K, U: the kept and the open rows among the 64 from the anchor's tile on
+        uint64_t K = 0, U = 0;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          // ---- anchors: the tile in x; candidates: x and y ----
+          const float ny = band_norm<DT>(y, ql, hl);
+          if (lane < 32) {
+            s_norm[wid][0][ql] = COS ? __builtin_amdgcn_rsqf(nx + 1e-8f) : nx;
+            s_norm[wid][1][ql] = COS ? __builtin_amdgcn_rsqf(ny + 1e-8f) : ny;
+          }
+          const float na = COS ? __builtin_amdgcn_rsqf(nx + 1e-8f) : nx;
+          constexpr uint32_t huge = 0x7b800000u;  // 2^120
+          const bool bad = (__float_as_uint(nx) & 0x7fffffffu) >= huge;
+          const uint32_t bad0 = (uint32_t)__ballot(bad);
+          const uint32_t bad1 = (uint32_t)__ballot((__float_as_uint(ny) & 0x7fffffffu) >= huge);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+          // S^T layout: the lane holds anchor ql and candidates 8 q + 4 hl + i of each tile
+          uint32_t kept[2], open[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const f32x16 g = band_gram<DT>(j == 0 ? x : y, x);
+            uint32_t kb = 0, db = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const f32x4 nc4 = *(const f32x4*)(&s_norm[wid][j][8 * q + 4 * hl]);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float dot = g[4 * q + i];
+                const uint32_t bit = 1u << (8 * q + i);
+                if (COS) {
+                  const float sim = dot * (na * nc4[i]);
+                  kb |= sim < bounds.keep ? bit : 0u;
+                  db |= sim > bounds.drop ? bit : 0u;
+                } else {
+                  const float n2 = na + nc4[i];
+                  kb |= __builtin_fmaf(n2, bounds.c_lo, -2.0f * dot) > bounds.keep ? bit : 0u;
+                  db |= __builtin_fmaf(n2, bounds.c_hi, -2.0f * dot) < bounds.drop ? bit : 0u;
+                }
+              }
+            }
+            kb <<= 4 * hl;
+            db <<= 4 * hl;
+            kb |= __shfl_xor(kb, 32, 64);
+            db |= __shfl_xor(db, 32, 64);
+            // candidates of this tile: after the anchor, before the chunk's end
+            const int lim = e - (tb + 32 * half + 32 * j);
+            uint32_t valid = lim >= 32 ? ~0u : lim > 0 ? (1u << lim) - 1u : 0u;
+            if (j == 0) valid &= ~((2u << ql) - 1u);
+            const uint32_t sure = bad ? 0u : ~(j == 0 ? bad0 : bad1);
+            kept[j] = kb & valid & sure;
+            open[j] = ~((kb | db) & sure) & valid;
+            __builtin_amdgcn_sched_barrier(0);  // one Gram tile's registers at a time
+          }
+          __builtin_amdgcn_wave_barrier();  // the norms are read before the next tile's are written
+          if (half == 0) {
+            x = y;
+            nx = ny;
+            load_tile(y, tb + 64);
+          }
+          if (hl == half) {  // lane l ends with row tb + l
+            K = kept[0] | (uint64_t)kept[1] << 32;
+            U = open[0] | (uint64_t)open[1] << 32;
+          }
+        }
+        // ---- exact decisions, until every anchor's first candidate is a kept one ----
+        const bool mine = tb + lane >= cur && tb + lane < e;
+        for (int round = 0; round < kBandRounds; ++round) {
+          const uint64_t any = K | U;
+          const int first = any ? __builtin_ctzll(any) : 0;
+          uint64_t m = __ballot(mine && any != 0 && ((U >> first) & 1ull));
+          if (m == 0) break;
+          int l[2 * kBandEval];
+          Row ra[kBandEval], rx[kBandEval];
+          uint64_t kp[kBandEval];
+#pragma unroll
+          for (int i = 0; i < 2 * kBandEval; ++i) {
+            l[i] = m ? __builtin_ctzll(m) : l[i > 0 ? i - 1 : 0];
+            m &= m - 1ull;
+          }
+#pragma unroll
+          for (int i = 0; i < kBandEval; ++i) {
+            const int f0 = (l[2 * i] & 32) + __builtin_amdgcn_readlane(first, l[2 * i]);
+            const int f1 = (l[2 * i + 1] & 32) + __builtin_amdgcn_readlane(first, l[2 * i + 1]);
+            ra[i] = row_bits(tb + (hl ? l[2 * i + 1] : l[2 * i]));
+            rx[i] = row_bits(tb + (hl ? f1 : f0));
+          }
+#pragma unroll
+          for (int i = 0; i < kBandEval; ++i) kp[i] = __ballot(half_keep<COS, A16, DT>(rx[i], ra[i], thr));
+#pragma unroll
+          for (int i = 0; i < 2 * kBandEval; ++i)
+            if (lane == l[i]) {
+              U &= ~(1ull << first);
+              if ((kp[i >> 1] >> (32 * (i & 1))) & 1ull) K |= 1ull << first;
+            }
+        }
+        // ---- the chain inside the wave's 64 rows, from every row at once: path holds the
+        // anchors met from row l on, to is where it leaves them (64 ..), or 128 + the anchor
+        // it stops at: one whose next is not known, to be looked for from row s_from on.
+        // Six doublings cover 64 steps. ----
+        const uint64_t any = K | U;
+        const int first = any ? __builtin_ctzll(any) : 64;
+        s_from[64 * wid + lane] = (uint8_t)((lane & 32) + first);
+        int to = any && !((U >> (first & 63)) & 1ull) ? (lane & 32) + first : 128 + lane;
+        uint32_t lo = lane < 32 ? 1u << ql : 0u, hi = lane < 32 ? 0u : 1u << ql;
+#pragma unroll
+        for (int d = 0; d < 6; ++d) {
+          const int src = to < 64 ? to : lane;
+          lo |= (uint32_t)__shfl((int)lo, src, 64);
+          hi |= (uint32_t)__shfl((int)hi, src, 64);
+          to = __shfl(to, src, 64);
+        }
+        s_path[64 * wid + lane] = u32x2{lo, hi};
+        s_to[64 * wid + lane] = (uint8_t)to;
+      }
+      __syncthreads();
+      if (wid == 0) {
+        // ---- the segment's chain: one lookup a block of 64 rows ----
+        int p = cur - sb;
+        for (int i = 0; i < seg / 64; ++i) {
+          uint64_t bits = 0;
+          while (p < 64 * (i + 1) && sb + p < se) {
+            const u32x2 path = s_path[p];
+            const int to = __builtin_amdgcn_readfirstlane((int)s_to[p]);
+            const uint64_t on = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(path[0]) |
+                                (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(path[1]) << 32;
+            bits |= on;
+            count += __builtin_popcountll(on);
+            if (to >= 128) {
+              // on from the anchor it stops at with the exact tree
+              const int pa = 64 * i + (to - 128);
+              const Row ra = row_bits(sb + pa);
+              int r = sb + 64 * i + __builtin_amdgcn_readfirstlane((int)s_from[pa]), at = e;
+              for (; r < e && at == e; r += 2 * kBandEval) {
+                Row rx[kBandEval];
+#pragma unroll
+                for (int u = 0; u < kBandEval; ++u) rx[u] = row_bits(min(r + 2 * u + hl, e - 1));
+#pragma unroll
+                for (int u = kBandEval - 1; u >= 0; --u) {  // the first of these rows that is kept
+                  const uint64_t kp = __ballot(half_keep<COS, A16, DT>(rx[u], ra, thr) && r + 2 * u + hl < e);
+                  if (kp) at = r + 2 * u + ((kp & 1ull) ? 0 : 1);
+                }
+              }
+              p = at - sb;
+            } else {
+              p = 64 * i + to;
+            }
+          }
+          if (lane == 0) s_bits[i] = bits;
+        }
+        if (lane == 0) s_cur = sb + p;
+      }
+      __syncthreads();
+      cur = __builtin_amdgcn_readfirstlane(s_cur);
+    } else {
+      if (tid < seg / 64) s_bits[tid] = 0;
+      __syncthreads();
+    }
+    if (sb + tid < se) keep_row[sb + tid] = (int32_t)((s_bits[tid >> 6] >> lane) & 1ull);
+    __syncthreads();  // the bits are read before the next segment's are written
+  }
+  if (tid == 0) chunk_counts[w] = count;  // tritonModules.py:68-69
+}
+
 static int launch_select(const void* k, int dtype, int64_t B, int64_t Hkv, int64_t N, int64_t D, int64_t sk_b,
                          int64_t sk_h, int64_t sk_n, float threshold, bool use_cosine, bool a16, int64_t chunk_size,
                          int64_t num_chunks, int32_t* keep, int32_t* chunk_counts, SeqMap seq, int64_t keep_sh,
@@ -311,6 +738,47 @@ static int launch_select(const void* k, int dtype, int64_t B, int64_t Hkv, int64
   const int64_t total = B * Hkv * num_chunks;
   const int64_t blocks = (total + 3) / 4;
   DA_REQUIRE(blocks < (1ll << 31), "%s: too many chunks", who);
+  // The banded walk takes rows it can read 16 bytes at a time.  It spends a workgroup of a
+  // wave per 64 rows on a chunk, two or more at once on a CU, so its time grows with the
+  // chunks where the serial walks stay at 0.14 us a row until the SIMDs are full: the line
+  // lies where the times meet, at two rounds of the chip (bf16, 8 heads: 64 chunks of 512
+  // rows a head 23 against 71 us, 128 a head 50 against 77, 192 a head 79 against 76 at one
+  // key in eight kept; fp32 keys, which take a CU each: 64 a head 37 against 62, 128 a head
+  // 79 against 70; cosine: 240 a head 96 against 140).  Below 96 rows a chunk is too short
+  // to gain (64 rows: 24 against 20 us).
+  const int per16 = dtype == DA_F32 ? 4 : 8;
+  const int64_t rows = seq.cu && divide_to > 0 ? (N + divide_to - 1) / divide_to : std::min(chunk_size, N);
+  const int64_t band_max = (dtype == DA_F32 ? 512 : use_cosine ? 2048 : 1024) * std::max<int64_t>(1, kBandSeg / rows);
+  if (rows >= kBandMinRows && total <= band_max && (D & 7) == 0 && ((sk_b | sk_h | sk_n) % per16) == 0 &&
+      ((uintptr_t)k & 15) == 0 && std::isfinite(threshold)) {
+    const BandBounds bounds = band_bounds(use_cosine, a16, dtype, threshold);
+    const unsigned threads = (unsigned)std::min<int64_t>(kBandSeg, (rows + 63) / 64 * 64);
+#define DA_BAND_LAUNCH_D(COS, A16, DT, FULL)                                                                  \
+  hipLaunchKernelGGL((select_band_kernel<COS, A16, DT, FULL>), dim3((unsigned)total), dim3(threads), 0, st, \
+                     (const uint16_t*)k, sk_b, sk_h, sk_n, (int)Hkv, N, (int)D,                            \
+                     (int)std::min<int64_t>(chunk_size, N), (int)num_chunks, threshold, bounds, keep,          \
+                     chunk_counts, seq, keep_sh, divide_to)
+#define DA_BAND_LAUNCH(COS, A16, DT)                                \
+  do {                                                              \
+    if (D == 128) DA_BAND_LAUNCH_D(COS, A16, DT, true);             \
+    else DA_BAND_LAUNCH_D(COS, A16, DT, false);                     \
+  } while (0)
+    if (dtype == DA_F32) {
+      if (use_cosine) DA_BAND_LAUNCH(true, false, DA_F32);
+      else DA_BAND_LAUNCH(false, false, DA_F32);
+    } else if (dtype == DA_F16) {
+      if (use_cosine) DA_BAND_LAUNCH(true, false, DA_F16);
+      else if (a16) DA_BAND_LAUNCH(false, true, DA_F16);
+      else DA_BAND_LAUNCH(false, false, DA_F16);
+    } else {
+      if (use_cosine) DA_BAND_LAUNCH(true, false, DA_BF16);
+      else if (a16) DA_BAND_LAUNCH(false, true, DA_BF16);
+      else DA_BAND_LAUNCH(false, false, DA_BF16);
+    }
+#undef DA_BAND_LAUNCH
+#undef DA_BAND_LAUNCH_D
+    return check_launch(who);
+  }
   if (dtype == DA_F32) {
     // fp32 keys: one wave per chunk, each lane two fp32 elements; the 16-bit definition
     // does not apply (the keys' own arithmetic is fp32)

@@ -528,3 +528,45 @@ def test_attention_with_sequence_stride_past_2_pow_22(gpu):
                                 p["counts"], W)
     _close(out_h.float().cpu().numpy(), want_h, "hybrid, stride 2^22+8")
     del kbuf, vbuf, kpbuf, vpbuf
+
+
+def _band_keys(kind, H, N, D, dtype):
+    gen = torch.Generator().manual_seed(N + D)
+    if kind == "equidistant":     # every pair at the same distance, 1.5 % from the threshold
+        k = torch.zeros((1, H, N, D))
+        k[0, :, torch.arange(N), torch.arange(N) % D] = 4.0
+    elif kind == "constant":      # no key past a chunk's first is kept
+        k = torch.randn((1, H, 1, D), generator=gen).expand(1, H, N, D)
+    elif kind == "slow":          # few keys kept, far apart
+        k = torch.randn((1, H, N, D), generator=gen).mul(0.05).cumsum(2)
+    elif kind == "huge":          # norms past fp32's range beside ordinary rows
+        k = torch.randn((1, H, N, D), generator=gen)
+        k[:, :, 5::7] *= 1e20 if dtype != torch.float16 else 3e3
+    else:
+        k = torch.randn((1, H, N, D), generator=gen)
+    return k.to(dtype).contiguous()
+
+
+@pytest.mark.parametrize("kind,H,N,D,chunk,metric,tau", [
+    ("equidistant", 2, 1100, 128, 512, "euclidean", 5.6), ("equidistant", 2, 1100, 128, 512, "euclidean", 5.75),
+    ("constant", 2, 1500, 128, 512, "euclidean", 0.5), ("slow", 2, 2100, 128, 1100, "euclidean", 4.0),
+    ("huge", 2, 700, 128, 300, "euclidean", 15.0), ("random", 3, 545, 96, 97, "euclidean", 13.5),
+    ("random", 2, 545, 8, 545, "euclidean", 4.0), ("random", 2, 577, 128, 128, "euclidean", 1e-20),
+    ("random", 2, 1300, 40, 0, "cosine", 0.1), ("slow", 2, 2100, 64, 700, "cosine", 0.99),
+    ("huge", 2, 700, 128, 300, "cosine", 0.1)])
+@pytest.mark.parametrize("dtype,arith", [(torch.bfloat16, "native"), (torch.bfloat16, "fp32"),
+                                         (torch.float16, "native"), (torch.float32, "native")],
+                         ids=["bf16", "bf16-fp32", "fp16", "fp32"])
+def test_select_banded_walk(gpu, kind, H, N, D, chunk, metric, tau, dtype, arith):
+    """The banded walk against the C oracle, bit for bit, where its shortcuts end: pairs all
+    close to the threshold, anchors whose next lies past the tiles compared, rows its bounds
+    do not hold for, chunk lengths around its tiles and segments, every key type."""
+    from deltaattention_amd import ops
+    k = _band_keys(kind, H, N, D, dtype)
+    announce(f"banded select {kind} H={H} N={N} D={D} chunk={chunk} {metric} tau={tau} {dtype} {arith}")
+    keep, cc = ops.select(k.to(gpu), tau, chunk, 2 if chunk == 0 else 0, metric, arith=arith)
+    orac = "fp32" if arith == "fp32" else oracle_arith(k)
+    ok, occ = OC.select_delta(k.float().numpy(), tau, chunk, 2 if chunk == 0 else 0, metric, arith=orac)
+    got = keep.cpu().numpy()
+    assert np.array_equal(got, ok), np.argwhere(got != ok)[:5]
+    assert np.array_equal(cc.cpu().numpy(), occ)
