@@ -5,13 +5,11 @@
 // hybrid_compressed_flash_kernel / _sanity / pure_phase1_flash_kernel
 // (deltaFlashAttention.py:9-357) with their wrappers (modeling_llama.py:306-451).
 //
-// Work decomposition.  A workgroup is 4 waves; each wave owns 32 query rows of one
-// query head.  The 4 waves always read the same KV head: with a GQA group of 4 they
-// are the 4 query heads of the group on the same 32 rows, so every K/V tile staged
-// in LDS serves 4 heads (repeat_kv is never materialised).  With smaller groups the
-// waves split 64 or 128 rows instead.  The rows of a workgroup lie inside one
-// logical 128-row query block of the reference, so the whole workgroup follows the
-// reference's schedule for that block.
+// Work decomposition.  A workgroup is 4 waves; each wave owns 64 query rows of one query
+// head.  The 4 waves always read the same KV head: with a GQA group of 4 they are 4 query
+// heads of the group on the same 64 rows, so every K/V tile staged in LDS serves 4 heads
+// (repeat_kv is never materialised).  With smaller groups the waves split 128 or 256 rows
+// instead.
 //
 // Logical schedule (deltaFlashAttention.py:58-113).  Phase 1 takes packed blocks of
 // 128 anchors while their maximum timestamp is < start_m - W; Phase 2 covers dense
@@ -25,17 +23,10 @@
 // v_mfma_f32_32x32x16_bf16 (the _f16 form for fp16 tensors; the kernels are templated on
 // the 16-bit type, and P is rounded to it as the reference rounds p to V's type): K
 // (32 keys x 16 dims) comes from LDS as the A operand,
-// Q^T stays in registers as the B operand for the whole key loop.  In the S^T
-// accumulator a lane holds one query and 16 keys, so the row max and row sum of the
-// online softmax are mostly in-lane (one exchange with lane ^ 32 per tile).  The
-// output is accumulated transposed too, O^T += V^T P^T: the 16-bit probabilities are
-// already in the B-operand layout, and V^T comes from an LDS tile that the loader
-// transposes while staging it.
-//
-// Pipeline.  Tiles of 64 keys (K: 16 KiB, V^T: 16 KiB, counts and timestamps:
-// 512 B) are double-buffered in LDS; the global loads of tile t+1 are issued before
-// tile t is computed and written to the other buffer afterwards, with one barrier
-// per tile.  Two workgroups fit per CU (66.5 KiB LDS each).
+// Q^T is the B operand for the whole key loop.  In the S^T accumulator a lane holds one
+// query and 16 keys, so the row sum of the online softmax is in-lane.  The output is
+// accumulated transposed too, O^T += V^T P^T: the 16-bit probabilities are already in the
+// B-operand layout, and V^T is read from the row-major V tile with transposing LDS reads.
 //
 // Softmax numerics.  exp2 with the softmax scale folded in: p = 2^(s*c - m*c) with
 // c = scale * log2(e) -- the same values as exp(s*scale - m*scale).  In Phase 1
@@ -52,10 +43,6 @@
 namespace da {
 
 constexpr int kD = 128;
-constexpr int kTileN = 64;
-constexpr int kKBytes = kTileN * kD * 2;
-constexpr int kVBytes = kD * kTileN * 2;
-constexpr int kStageBytes = kKBytes + kVBytes + kTileN * 4 + kTileN * 4;
 constexpr int kBlock = 128;  // logical block of the reference schedule
 
 enum Variant : int { kHybrid = 0, kSanity = 1, kPure = 2, kDense = 3 };
@@ -89,112 +76,20 @@ struct AttnArgs {
   int causal;
   const int32_t* sched;  // [B*Hkv][2][nblk_cap]: block maxima, prefix maxima
   int nblk_cap;
-  // prepared by the schedule kernel for the ping-pong kernel, [B*Hkv][wcap] each:
+  // prepared by the schedule kernel, [B*Hkv][wcap] each:
   const float* wts;    // key bias log2(w_i) / scale_log2 of packed row i (-inf where w_i = 0)
   const int32_t* tsw;  // timestamp of packed row i, INT_MAX where the weight is 0
   const float* zeros;  // 64 zero biases (the exact tiles)
   int wcap;            // nblk_cap * 128
   int hpw;          // query heads per workgroup (4, 2 or 1)
-  int rows_per_wg;  // 32 * (4 / hpw)
+  int rows_per_wg;  // 256 / hpw
   int n_row_groups;
   int units;        // B * Hkv * (G / hpw)
+  int slots;        // workgroups an XCD runs at once, two a CU
   int* queue;       // 8 work-queue counters (persistent attn_w64_kernel grid) or null
 };
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// LDS byte offsets inside a stage.
-__device__ __forceinline__ int k_lds_off(int row, int chunk) {
-  return row * (kD * 2) + ((chunk ^ (row & 15)) << 4);
-}
-// V^T rows (one per head dimension) hold the 64 keys of the tile permuted so that
-// the 8 keys one lane feeds to a P.V MFMA -- keys 16u + 4h + {0..3} and
-// 16u + 8 + 4h + {0..3} -- form 16-byte chunk 2u + h.  A group of 4 consecutive keys
-// 4kg..4kg+3 is the 8-byte half (kg >> 1) & 1 of chunk 2 (kg >> 2) + (kg & 1).
-// Chunks are XOR-swizzled with (d & 7) ^ ((d >> 3) & 1) so that 8 (or 16) consecutive
-// rows read at one chunk index hit distinct banks.
-__device__ __forceinline__ int vt_swz(int d) { return (d & 7) ^ ((d >> 3) & 1); }
-__device__ __forceinline__ int vt_lds_chunk(int d, int chunk) {
-  return kKBytes + d * (kTileN * 2) + ((chunk ^ vt_swz(d)) << 4);
-}
-__device__ __forceinline__ int vt_lds_group(int d, int kg) {
-  return vt_lds_chunk(d, 2 * (kg >> 2) + (kg & 1)) + (((kg >> 1) & 1) << 3);
-}
-constexpr int kCntOff = kKBytes + kVBytes;
-constexpr int kTsOff = kCntOff + kTileN * 4;
-
-struct TileRegs {
-  u32x4 k[4];
-  u32x4 v[4];
-  float cnt;
-  int ts;
-};
-
-// Global -> registers for one 64-key tile.  For K, thread tid loads 16-byte chunk
-// (tid % 16) of keys 4 * (tid / 16) + j, j = 0..3 (a wave writes whole 256-byte K
-// rows).  For V the roles swap -- chunk tid / 16 of keys 4 * (tid % 16) + j -- so that
-// after the in-register transpose the 16 lanes of one chunk write one complete
-// 128-byte V^T row, which keeps the LDS stores free of bank conflicts.
-__device__ __forceinline__ void load_tile(TileRegs& r, const uint16_t* kbase, const uint16_t* vbase,
-                                          int64_t sk_n, int64_t sv_n, int key0, int limit, int D,
-                                          int tid, bool with_meta, const int32_t* tsrow,
-                                          const void* cntrow, int cnt_is_float, int no_count,
-                                          int meta_limit, int ts_oob) {
-  const int chunk = tid & 15, kg = tid >> 4;    // K mapping
-  const int vchunk = tid >> 4, vkg = tid & 15;  // V mapping
-  // 8-dim chunks at or beyond the head dimension are zero (BLOCK_D padding of the reference)
-  const bool kin = chunk * 8 < D, vin = vchunk * 8 < D;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int key = key0 + kg * 4 + j;
-    r.k[j] = (kin && key < limit) ? *(const u32x4*)(kbase + (int64_t)key * sk_n + chunk * 8)
-                                  : u32x4{0, 0, 0, 0};
-    const int vkey = key0 + vkg * 4 + j;
-    r.v[j] = (vin && vkey < limit) ? *(const u32x4*)(vbase + (int64_t)vkey * sv_n + vchunk * 8)
-                                   : u32x4{0, 0, 0, 0};
-  }
-  if (with_meta && tid < kTileN) {
-    const int key = key0 + tid;
-    if (key < meta_limit) {
-      if (no_count)
-        r.cnt = 1.0f;
-      else if (cnt_is_float)
-        r.cnt = ((const float*)cntrow)[key];
-      else
-        r.cnt = (float)((const int32_t*)cntrow)[key];
-      r.ts = tsrow ? tsrow[key] : 0;
-    } else {
-      r.cnt = 0.0f;
-      r.ts = ts_oob;
-    }
-  }
-}
-
-__device__ __forceinline__ void store_tile(const TileRegs& r, char* stage, int tid, bool with_meta) {
-  const int chunk = tid & 15, kg = tid >> 4;
-  const int vchunk = tid >> 4, vkg = tid & 15;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) *(u32x4*)(stage + k_lds_off(kg * 4 + j, chunk)) = r.k[j];
-  // transpose 4 keys x 8 dims into 8 rows (dims) of 4 keys
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const uint32_t a = r.v[0][w], b = r.v[1][w], c = r.v[2][w], d = r.v[3][w];
-    const int d0 = vchunk * 8 + 2 * w;
-    // v_perm_b32 picks bytes of {S0 = high word, S1 = low word}: 0x05040100 gives
-    // (lo16(a), lo16(b)), 0x07060302 gives (hi16(a), hi16(b)).
-    u32x2 lo, hi;
-    lo[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
-    lo[1] = __builtin_amdgcn_perm(d, c, 0x05040100u);
-    hi[0] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-    hi[1] = __builtin_amdgcn_perm(d, c, 0x07060302u);
-    *(u32x2*)(stage + vt_lds_group(d0, vkg)) = lo;
-    *(u32x2*)(stage + vt_lds_group(d0 + 1, vkg)) = hi;
-  }
-  if (with_meta && tid < kTileN) {
-    ((float*)(stage + kCntOff))[tid] = r.cnt;
-    ((int*)(stage + kTsOff))[tid] = r.ts;
-  }
-}
 
 // Phase-1 extent of a query block (deltaFlashAttention.py:58-80): n_safe = the number of
 // packed blocks whose prefix maximum timestamp is below thr -- the prefix maxima do not
@@ -230,256 +125,6 @@ __device__ __forceinline__ void safe_prefix(const int32_t* __restrict__ bmax, co
     prev_last = last;
   }
   n_safe = n;
-}
-
-template <int VARIANT, int DT>
-__device__ __forceinline__ void attn_body(const AttnArgs& a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
-  const int hl = lane >> 5;   // which half of the wave
-  const int ql = lane & 31;   // query column of this lane
-
-  // ---- workgroup -> (unit, row group): XCD-aware, longest rows first ----
-  const int wg = blockIdx.x;
-  int unit, rg;
-  if ((a.units & 7) == 0) {
-    // workgroup i runs on XCD i mod 8; each XCD takes whole units (a KV head of one
-    // sequence) and runs them one after another, every unit's row groups longest first,
-    // so the 32 CUs of an XCD share one unit's K/V in their L2
-    const int xcd = wg & 7, idx = wg >> 3, upx = a.units >> 3;
-    unit = xcd * upx + idx / a.n_row_groups;
-    rg = a.n_row_groups - 1 - idx % a.n_row_groups;
-  } else {
-    unit = wg % a.units;
-    rg = a.n_row_groups - 1 - wg / a.units;
-  }
-  // units are KV-head major, so that the XCD mapping above gives each XCD whole KV
-  // heads of every sequence (balanced when the sequences of a batch differ in length)
-  const int hunits = a.G / a.hpw;
-  const int gb = unit / hunits;  // g * B + b
-  const int hu = unit - gb * hunits;
-  const int g = gb / a.B, b = gb - (gb / a.B) * a.B;
-  const int bg = b * a.Hkv + g;
-  const int h = g * a.G + hu * a.hpw + (wid % a.hpw);
-  const int R0 = rg * a.rows_per_wg;
-  const int Nq = a.seq.cu ? a.seq.len(b) : a.Nq;
-  const int Nk = a.seq.cu ? a.seq.len(b) : a.Nk;
-  if (R0 >= Nq) return;  // a row group past the end of a shorter sequence (whole workgroup)
-  const int r0w = R0 + (wid / a.hpw) * 32;  // first row of this wave
-  const int wg_end = R0 + a.rows_per_wg;    // one past the last row of the workgroup
-  const int start_m = (R0 / kBlock) * kBlock;
-
-  // ---- schedule ----
-  int P = a.P_host;
-  if (a.P_dev) P = min(a.seq.cu ? a.P_dev[b] : *a.P_dev, a.P_host);
-  if (a.seq.cu) P = min(P, Nk);  // a sequence's packed rows lie inside its own tokens
-  int n1 = 0, ds = 0;
-  int kend = a.causal ? min(Nk, wg_end) : Nk;
-  if (VARIANT == kHybrid || VARIANT == kSanity) {
-    const int nblk = (P + kBlock - 1) / kBlock;
-    const int32_t* bmax = a.sched + (int64_t)bg * 2 * a.nblk_cap;
-    const int32_t* pmax = bmax + a.nblk_cap;
-    int n_safe, last;
-    safe_prefix(bmax, pmax, nblk, start_m - a.window, n_safe, last, lane);
-    ds = max(0, ((last + 1) / kBlock) * kBlock);
-    if (VARIANT == kHybrid) n1 = n_safe * (kBlock / kTileN);
-    kend = min(Nk, wg_end);
-  } else if (VARIANT == kPure) {
-    n1 = (P + kTileN - 1) / kTileN;
-    kend = 0;
-  }
-  const int n2 = kend > ds ? (kend - ds + kTileN - 1) / kTileN : 0;
-  const int ntiles = n1 + n2;
-
-  const uint16_t* kp_base = a.kp + a.seq.base(b, a.skp_b, a.skp_n) + (int64_t)g * a.skp_h;
-  const uint16_t* vp_base = a.vp + a.seq.base(b, a.svp_b, a.svp_n) + (int64_t)g * a.svp_h;
-  const uint16_t* k_base = a.k + a.seq.base(b, a.sk_b, a.sk_n) + (int64_t)g * a.sk_h;
-  const uint16_t* v_base = a.v + a.seq.base(b, a.sv_b, a.sv_n) + (int64_t)g * a.sv_h;
-  const int32_t* ts_row = a.ts ? a.ts + a.seq.base(b, a.sts_b, 1) + (int64_t)g * a.sts_h : nullptr;
-  const char* cnt_row = a.cnt ? (const char*)a.cnt + (a.seq.base(b, a.scnt_b, 1) + (int64_t)g * a.scnt_h) * 4 : nullptr;
-  const bool meta = (VARIANT == kHybrid || VARIANT == kPure);
-
-  // ---- Q^T in registers (B operand): lane (ql, hl) holds dims 16t + 8hl .. +7 ----
-  u32x4 qreg[kD / 16];
-  {
-    const int row = r0w + ql;
-    const uint16_t* qrow = a.q + a.seq.base(b, a.sq_b, a.sq_n) + (int64_t)h * a.sq_h + (int64_t)row * a.sq_n;
-#pragma unroll
-    for (int t = 0; t < kD / 16; ++t)
-      qreg[t] = (row < Nq && 16 * t + 8 * hl < a.D) ? *(const u32x4*)(qrow + 16 * t + 8 * hl)
-                                                       : u32x4{0, 0, 0, 0};
-  }
-
-  f32x16 o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = f32x16{};
-  float m_i = -INFINITY, l_i = 0.0f;
-  const float c = a.scale_log2;
-
-  TileRegs regs;
-  auto tile_src = [&](int t, const uint16_t*& kb, const uint16_t*& vb, int64_t& skn, int64_t& svn,
-                      int& key0, int& limit, bool& ph1) {
-    ph1 = t < n1;
-    if (ph1) {
-      kb = kp_base; vb = vp_base; skn = a.skp_n; svn = a.svp_n; key0 = t * kTileN; limit = P;
-    } else {
-      kb = k_base; vb = v_base; skn = a.sk_n; svn = a.sv_n; key0 = ds + (t - n1) * kTileN; limit = Nk;
-    }
-  };
-
-  if (ntiles > 0) {
-    const uint16_t *kb, *vb; int64_t skn, svn; int key0, limit; bool ph1;
-    tile_src(0, kb, vb, skn, svn, key0, limit, ph1);
-    load_tile(regs, kb, vb, skn, svn, key0, limit, a.D, tid, meta && ph1, ts_row, cnt_row,
-              a.cnt_is_float, a.no_count, P, Nk + 1);
-    store_tile(regs, smem, tid, meta && ph1);
-  }
-  __syncthreads();
-
-  for (int t = 0; t < ntiles; ++t) {
-    char* stage = smem + (t & 1) * kStageBytes;
-    const bool has_next = t + 1 < ntiles;
-    bool next_ph1 = false;
-    if (has_next) {
-      const uint16_t *kb, *vb; int64_t skn, svn; int key0, limit;
-      tile_src(t + 1, kb, vb, skn, svn, key0, limit, next_ph1);
-      load_tile(regs, kb, vb, skn, svn, key0, limit, a.D, tid, meta && next_ph1, ts_row, cnt_row,
-                a.cnt_is_float, a.no_count, P, Nk + 1);
-    }
-
-    const bool ph1 = t < n1;
-    const int key0 = ph1 ? t * kTileN : ds + (t - n1) * kTileN;
-    // wave-uniform skip of tiles entirely above this wave's rows (causal)
-    const bool skip = !ph1 && a.causal && key0 > r0w + 31;
-    if (!skip) {
-      // ---- S^T = K Q^T for two 32-key blocks ----
-      // the two key blocks alternate so that consecutive MFMAs do not depend on each other
-      f32x16 s[2] = {f32x16{}, f32x16{}};
-#pragma unroll
-      for (int tt = 0; tt < kD / 16; ++tt) {
-#pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2) {
-          const u32x4 w = *(const u32x4*)(stage + k_lds_off(kb2 * 32 + ql, 2 * tt + hl));
-          s[kb2] = E16<DT>::mfma(w, qreg[tt], s[kb2]);
-        }
-      }
-      // ---- masks ----
-      const int row = r0w + ql;
-      if (VARIANT == kPure) {
-        const float* cl = (const float*)(stage + kCntOff);
-        const int* tl = (const int*)(stage + kTsOff);
-#pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kl = kb2 * 32 + 8 * (r >> 2) + 4 * hl + (r & 3);
-            const bool ok = cl[kl] > 0.0f && tl[kl] <= row;  // deltaFlashAttention.py:321-330
-            if (!ok) s[kb2][r] = -INFINITY;
-          }
-      } else if (!ph1) {
-        const bool need = (a.causal && key0 + kTileN - 1 > r0w) || key0 + kTileN > Nk;
-        if (need) {
-#pragma unroll
-          for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int key = key0 + kb2 * 32 + 8 * (r >> 2) + 4 * hl + (r & 3);
-              const bool ok = key < Nk && (!a.causal || key <= row);
-              if (!ok) s[kb2][r] = -INFINITY;
-            }
-        }
-      }
-      // ---- online softmax ----
-      float mx = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, __builtin_fmaxf(s[0][r], s[1][r]));
-      mx = fmaxf(mx, swap_halves(mx));
-      const float m_new = fmaxf(m_i, mx);
-      const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-      const float alpha = exp2_fast((m_i - m_use) * c);
-      const float neg = -m_use * c;
-      // P^T as four B operands (16 keys each): operand u = 2 * kb2 + (r4 >> 1) holds
-      // S^T registers 8 * (r4 >> 1) .. +7 of block kb2.
-      u32x4 pw[4];
-      float psum = 0.0f;
-      const bool weighted = (VARIANT == kPure) || (VARIANT == kHybrid && ph1);
-      const float* cl = (const float*)(stage + kCntOff);
-#pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2) {
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          f32x4 w4 = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
-          if (weighted) w4 = *(const f32x4*)(cl + kb2 * 32 + 8 * r4 + 4 * hl);
-          float p[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            p[e] = exp2_fast(__builtin_fmaf(s[kb2][4 * r4 + e], c, neg));
-            if (weighted) p[e] *= w4[e];
-          }
-          psum += (p[0] + p[1]) + (p[2] + p[3]);
-          pw[2 * kb2 + (r4 >> 1)][(r4 & 1) * 2 + 0] = E16<DT>::pack(p[0], p[1]);
-          pw[2 * kb2 + (r4 >> 1)][(r4 & 1) * 2 + 1] = E16<DT>::pack(p[2], p[3]);
-        }
-      }
-      l_i = l_i * alpha + psum;
-      m_i = m_new;
-      if (__ballot(alpha != 1.0f)) {
-#pragma unroll
-        for (int db = 0; db < 4; ++db)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-      }
-      // ---- O^T += V^T P^T ----
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-          const int d = db * 32 + ql;
-          const u32x4 vw = *(const u32x4*)(stage + vt_lds_chunk(d, 2 * u + hl));
-          o[db] = E16<DT>::mfma(vw, pw[u], o[db]);
-        }
-      }
-    }
-    if (has_next) store_tile(regs, smem + ((t + 1) & 1) * kStageBytes, tid, meta && next_ph1);
-    __syncthreads();
-  }
-
-  // ---- finalize: out = acc / l ----
-  const float l_tot = l_i + swap_halves(l_i);
-  float inv;
-  if (VARIANT == kPure)
-    inv = l_tot > 0.0f ? 1.0f / l_tot : 1.0f;  // deltaFlashAttention.py:353-354
-  else
-    inv = 1.0f / l_tot;
-  const int row = r0w + ql;
-  if (row < Nq) {
-    uint16_t* orow = a.out + a.seq.base(b, a.so_b, a.so_n) + (int64_t)h * a.so_h + (int64_t)row * a.so_n;
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        u32x2 w;
-        w[0] = E16<DT>::pack(o[db][4 * j + 0] * inv, o[db][4 * j + 1] * inv);
-        w[1] = E16<DT>::pack(o[db][4 * j + 2] * inv, o[db][4 * j + 3] * inv);
-        if (db * 32 + 8 * j + 4 * hl < a.D) *(u32x2*)(orow + db * 32 + 8 * j + 4 * hl) = w;
-      }
-  }
-}
-
-// Per-head kernel entry points.  Dense, hybrid and sanity fit two waves per SIMD
-// (<= 256 registers).  The pure-Phase-1 body needs more: capped at 256 it spills, and that
-// build gave wrong pure-Phase-1 outputs on every row while the same source without the
-// cap (no spills) matches the oracle, so it runs at one wave per SIMD.
-template <int VARIANT, int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attn_kernel(AttnArgs a) {
-  attn_body<VARIANT, DT>(a);
-}
-template <int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
-void attn_kernel_pure(AttnArgs a) {
-  attn_body<kPure, DT>(a);
 }
 
 // min(max(x, 0), hi) for a wave-uniform x, kept in scalar registers (the compiler would
@@ -571,36 +216,42 @@ __device__ __forceinline__ float halves_sum(float x) {
 // s_waitcnt immediate (gfx9 encoding) that waits for vmcnt <= n only.
 constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
-// The 64-row kernel updates its running maximum lazily: only when a tile's maximum
+// The 16-bit kernel updates its running maximum lazily: only when a tile's maximum
 // exceeds it by more than 2^8 in probability (8 in log2 units) are O and l rescaled.
 constexpr float kLazyLog2 = 8.0f;
-// The 64-row kernel computes p against the current maximum before it looks at the
+// The 16-bit kernel computes p against the current maximum before it looks at the
 // tile's maximum, and needs the latter only where a lane's sum of its 16 p exceeds
 // 16 * 2^8: below that bound every p is at most 2^8 * 16, and a rescale is not needed
 // (p stays far from fp32's range and keeps bf16's relative precision).
 constexpr float kLazySum = 16.0f * 256.0f;
 
 // ====================================================================================
-// Ping-pong kernel for GQA groups that are a multiple of 4 (the Llama-3 hot path).
+// The 16-bit attention kernel, for every GQA group.
 //
-// A workgroup is 8 waves, two per SIMD, and covers one logical 128-row query block of
-// the reference's schedule for 4 query heads of one GQA group, so all 8 waves read the
-// same K/V tiles.  Waves 0-3 (group A) own rows R0..R0+63 and waves 4-7 (group B) rows
-// R0+64..R0+127, each wave one query head, as two 32-row column blocks.  Tiles are 32
-// keys; every tile boundary falls on the reference's logical 128-key grid.
+// A workgroup is 4 waves, one per SIMD: 4, 2 or 1 query heads of a GQA group (hpw) over 64,
+// 128 or 256 rows, each wave 64 rows of one head as two 32-row column blocks, so that every K
+// fragment and every V^T fragment read from LDS feeds two MFMAs.  Two workgroups share a CU:
+// while a wave runs its softmax (VALU), the other workgroup's wave on its SIMD has the matrix
+// pipe (its MFMAs go out at raised priority).  Tiles are 32 keys; every tile boundary falls
+// on the reference's logical 128-key grid.
 //
-// In every section one group runs its matrix work (P.V of the previous tile, then Q.K
-// of the current one: 32 MFMAs at raised issue priority) while the other group runs its
-// softmax (VALU); group B runs one section behind group A, so the two waves sharing a
-// SIMD have complementary work and the MFMA pipe and the VALU co-execute.  Two sections
-// form a window; the workgroup synchronises once per window.  Every K fragment and every
-// V^T fragment read from LDS feeds two MFMAs, one per column block.
+// A window is the matrix work of a wave's tile (P.V of the previous one, then Q.K), a
+// barrier, the loads of later tiles, the softmax.  K and V tiles go straight from memory to
+// LDS (buffer_load ... lds), two stages each, a window ahead of their use; V is kept row-major
+// and read as V^T with ds_read_b64_tr_b16.  No tile passes through registers.  Q of column
+// block 0 stays in registers; Q of column block 1 sits in LDS, lane-private (each lane reads
+// back only what it wrote), which keeps the wave within 256 registers and the workgroup's LDS
+// (66 KiB) within half a CU's.
 //
-// K and V tiles go straight from memory to LDS (buffer_load ... lds), three stages each,
-// issued two windows (K) and one window (V) ahead of their use; V is kept row-major and
-// read as V^T with ds_read_b64_tr_b16.  No tile passes through registers.  Q of column
-// block 0 stays in registers; Q of column block 1 sits in LDS, lane-private (each lane
-// reads back only what it wrote), which keeps the wave within 256 registers.
+// Against one 8-wave workgroup a CU (two such groups in lockstep, half a window apart), which
+// this replaces: items are half as long, so small grids end sooner (dense 1024 tokens x 32
+// heads 44 against 53 us, 2048 80 / 93, 4096 162 / 180), and an item's first loads, epilogue
+// and queue take run under the other workgroup's tiles (hybrid, one key in four: 32768 tokens
+// 1.97 against 2.04 ms, 131072 27.9 / 28.7; ragged batches 4.5 / 4.7 ms).  It reads each tile
+// twice as often from L2, which costs up to 0.3 % where neither matters (dense 32768).  Groups
+// that are not a multiple of 4 ran a 32-row kernel that staged tiles through registers: 8000
+// tokens x 32 heads, keys repeated to the query heads, 233 against 318 us; dense 16384 x 32
+// heads of their own 1.85 against 2.70 ms.
 // ====================================================================================
 constexpr int kWTK = 32;                         // keys per tile
 constexpr int kWKBytes = kWTK * kD * 2;          // 8 KiB
@@ -608,13 +259,14 @@ constexpr int kWVBytes = kWTK * kD * 2;          // 8 KiB
 constexpr int kWMetaSlot = 64 * 8;               // weights[64] fp32, timestamps[64] int32
 constexpr int kWCnt = 0, kWTs = 64 * 4;          // offsets inside a meta slot
 constexpr int kWQBytes = 32 * kD * 2;          // Q of one 32-row column block, per wave
-// the persistent grid's item broadcast (two ints) after the Q regions
-constexpr int kWItemSlot = 3 * kWKBytes + 3 * kWVBytes + 4 * kWMetaSlot + 8 * kWQBytes;
-constexpr int kWLds = kWItemSlot + 16;  // item: queue, index, queues found empty
+// LDS: two stages each of K and V, the weights' ring, the four waves' Q regions, then the
+// persistent grid's item broadcast (queue, index, queues found empty)
+constexpr int kWItemSlot = 2 * (kWKBytes + kWVBytes) + 4 * kWMetaSlot + 4 * kWQBytes;
+constexpr int kWLds = kWItemSlot + 16;
 // K stages and Q blocks start at multiples of 256 bytes (the kernel has no static LDS, so
 // its dynamic LDS starts at address 0): the K / Q fragment addresses are formed by XOR.
-static_assert(kWKBytes % 256 == 0 && (3 * kWKBytes + 3 * kWVBytes + 4 * kWMetaSlot) % 256 == 0 &&
-              kWQBytes % 256 == 0, "K stages and Q blocks must be 256-byte aligned");
+static_assert(kWKBytes % 256 == 0 && kWVBytes % 256 == 0 && (4 * kWMetaSlot) % 256 == 0 && kWQBytes % 256 == 0,
+              "K stages and Q blocks must be 256-byte aligned");
 
 // Masks of one 32-key x 32-row score block (S^T register r holds key 8 (r / 4) + 4 hl +
 // r % 4 of the tile for the lane's row).
@@ -644,16 +296,32 @@ __device__ __forceinline__ void queue_units(int q, int units, int& ulo, int& uhi
   uhi = ((q + 1) * units) >> 3;
 }
 
-// One (unit, row group) of attn_w64_kernel: 4 query heads of one (batch, KV head) over
-// the logical 128-row query block rg.  Ends with every LDS read of the window loop done
-// (its last barrier) and every load landed; the finalize uses only the wave's own Q
-// region, so the next item may start staging at once.
+// Item k of an XCD's n = units * n_rg (unit, row group) pairs: unit by unit, the longest row
+// groups first.  Where all of them start at once, two a CU, the first half of the slots takes
+// the longest, one a CU, and the rest run from the shortest up, so that every CU gets about
+// the same work.
+__device__ __forceinline__ void item_at(int k, int units, int n_rg, int slots, int& unit, int& rg) {
+  const int n = units * n_rg, half = slots >> 1;
+  if (n <= slots) {
+    const int e = k < half ? k : n - 1 - (k - half);
+    unit = e % units;
+    rg = n_rg - 1 - e / units;
+  } else {
+    unit = k / n_rg;
+    rg = n_rg - 1 - (k - unit * n_rg);
+  }
+}
+
+// One (unit, row group) of attn_w64_kernel: a.hpw (4, 2 or 1) query heads of one (batch, KV
+// head) over 256 / hpw rows.  Ends with every LDS read of the window loop done (its last
+// barrier) and every load landed; the finalize uses only the wave's own Q region, so the next
+// item may start staging at once.
 template <int VARIANT, int DT>
 __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit, const int rg) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* const kst0 = smem;
-  char* const vst0 = smem + 3 * kWKBytes;
-  char* const meta0 = smem + 3 * kWKBytes + 3 * kWVBytes;
+  char* const vst0 = smem + 2 * kWKBytes;
+  char* const meta0 = smem + 2 * (kWKBytes + kWVBytes);
   // opaque per item: what derives from the thread index is formed here, not hoisted out
   // of the persistent grid's item loop into registers held across items
   int tid = threadIdx.x;
@@ -663,41 +331,68 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   // Q of column block 1, lane-private: each lane reads back only the 16-byte chunks it
   // wrote (the K fragment layout), so the 32 registers it would take stay free
   char* const qs = meta0 + 4 * kWMetaSlot + wid * kWQBytes;
-  const int grp = wid >> 2, hw = wid & 3;
   const int hl = lane >> 5, ql = lane & 31;
-  const int hunits = a.G >> 2;
+  const int hsh = a.hpw >> 1;  // log2 of the query heads a workgroup takes
+  const int hunits = a.G >> hsh;
   const int gb = unit / hunits;  // g * B + b
   const int hu = unit - gb * hunits;
   const int g = gb / a.B, b = gb - (gb / a.B) * a.B;
   const int bg = b * a.Hkv + g;
-  const int h = g * a.G + hu * 4 + hw;
-  const int R0 = rg * 128;
+  const int h = g * a.G + (hu << hsh) + (wid & ((1 << hsh) - 1));
+  const int wg_rows = 256 >> hsh;
+  const int R0 = rg * wg_rows;
   const int Nq = a.seq.cu ? a.seq.len(b) : a.Nq;
   const int Nk = a.seq.cu ? a.seq.len(b) : a.Nk;
   if (R0 >= Nq) return;  // a row group past the end of a shorter sequence (whole workgroup)
-  const int r0w = R0 + grp * 64;  // first row of this wave; column block cb holds r0w + 32 cb + ql
-  const int wg_end = R0 + 128;
-  const int start_m = R0;
+  // first row of this wave; column block cb holds r0w + 32 cb + ql
+  const int r0w = R0 + 64 * (wid >> hsh);
+  const int wg_end = R0 + wg_rows;
 
-  // ---- schedule of the logical 128-row block R0 ----
+  // ---- schedule: packed tiles 0 .. n1 - 1, then exact tiles from key ds on.  A workgroup's
+  // rows lie in one logical 128-row block, except where one head takes 256 rows (hpw
+  // 1): its tiles are then the union of the two blocks' schedules, and a wave skips those
+  // that its own block (n1w, dsw) does not have ----
   int P = a.P_host;
   if (a.P_dev) P = min(a.seq.cu ? a.P_dev[b] : *a.P_dev, a.P_host);
   if (a.seq.cu) P = min(P, Nk);
-  int n1 = 0, ds = 0;
+  int n1 = 0, ds = 0, n1w = 0, dsw = 0;
   int kend = a.causal ? min(Nk, wg_end) : Nk;
   if (VARIANT == kHybrid || VARIANT == kSanity) {
     const int nblk = (P + kBlock - 1) / kBlock;
     const int32_t* bmax = a.sched + (int64_t)bg * 2 * a.nblk_cap;
     const int32_t* pmax = bmax + a.nblk_cap;
-    int n_safe, last;
-    safe_prefix(bmax, pmax, nblk, start_m - a.window, n_safe, last, lane);
-    ds = max(0, ((last + 1) / kBlock) * kBlock);
-    if (VARIANT == kHybrid) n1 = n_safe * (kBlock / kWTK);
+    auto block_schedule = [&](const int start_m, int& n, int& d) {
+      int n_safe, last;
+      safe_prefix(bmax, pmax, nblk, start_m - a.window, n_safe, last, lane);
+      d = max(0, ((last + 1) / kBlock) * kBlock);
+      n = VARIANT == kHybrid ? n_safe * (kBlock / kWTK) : 0;
+    };
+    // a wave past the last row follows the last block that has rows: every wave of the
+    // workgroup must come to the same tiles
+    const int start_w = min(r0w, Nq - 1) & ~(kBlock - 1);
+    block_schedule(start_w, n1w, dsw);
+    n1 = n1w;
+    ds = dsw;
+    if (hsh == 0 && R0 + kBlock < Nq) {
+      int n2w, d2w;
+      block_schedule(start_w ^ kBlock, n2w, d2w);
+      n1 = max(n1, n2w);
+      ds = min(ds, d2w);
+    }
     kend = min(Nk, wg_end);
   } else if (VARIANT == kPure) {
-    n1 = (P + kWTK - 1) / kWTK;
+    // the packed blocks up to the last that holds a key at or before the last row
+    const int nblk = (P + kBlock - 1) / kBlock;
+    const int32_t* from = a.sched + (int64_t)bg * 2 * a.nblk_cap + a.nblk_cap;
+    int last;
+    safe_prefix(from, from, nblk, r0w + 64, n1w, last, lane);
+    safe_prefix(from, from, nblk, wg_end, n1, last, lane);
+    n1w = min(n1w * (kBlock / kWTK), (P + kWTK - 1) / kWTK);
+    n1 = min(n1 * (kBlock / kWTK), (P + kWTK - 1) / kWTK);
     kend = 0;
   }
+  n1 = __builtin_amdgcn_readfirstlane(n1);
+  ds = __builtin_amdgcn_readfirstlane(ds);
   const int n2 = kend > ds ? (kend - ds + kWTK - 1) / kWTK : 0;
   const int T = n1 + n2;
 
@@ -718,12 +413,16 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     const int d = r0w + 63 - ds;
     t_skip = __builtin_amdgcn_readfirstlane(d < 0 ? n1 : n1 + d / kWTK + 1);
   }
-  auto skipped = [&](int t) { return t >= t_skip; };
+  if (kPureV) t_skip = __builtin_amdgcn_readfirstlane(n1w);
+  if (r0w >= Nq) t_skip = 0;  // no rows
+  // and those of the other logical block: [skip_lo, skip_hi)
+  const int skip_lo = __builtin_amdgcn_readfirstlane(n1w);
+  const int skip_hi = __builtin_amdgcn_readfirstlane(n1 + (dsw - ds) / kWTK);
 
-  // ---- staging: loads straight into LDS, three stages each for K and V and a ring of
-  // four slots for the tiles' weights.  Wave w loads rows 4w .. 4w + 3 of both tiles:
-  // lane l writes 16 bytes at 1 KiB w + 16 l, i.e. row 4w + l / 16 at position l % 16,
-  // so it fetches the source chunk that the swizzled layout keeps there.  The buffer
+  // ---- staging: loads straight into LDS, two stages each for K and V and a ring of
+  // four slots for the tiles' weights.  Wave w loads rows 8w .. 8w + 7 of both tiles in two
+  // steps of four: lane l writes 16 bytes at 1 KiB (2 w + j) + 16 l, i.e. row 8 w + 4 j + l / 16
+  // at position l % 16, so it fetches the source chunk that the swizzled layout keeps there.  The buffer
   // resource covers exactly the tile's valid keys: rows past the end, and 8-dim chunks
   // at or beyond the head dimension, arrive as zeros.  Each wave issues the same loads
   // in every window, so the s_waitcnt vmcnt(n) at the end of a window, n = the loads of
@@ -749,15 +448,19 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(base), (short)0, range, kBufferDword3);
     char* dst = isK ? kst0 + st : vst0 + st;
-    const int rowt = wid_s * 4 + (lane >> 4);
-    const int pos = lane & 15;
-    const int chunk = pos ^ (isK ? (rowt & 15) : 4 * (rowt & 3));
-    // rowt < 32 and snb < 2^24 (the host limits sequence strides to 2^23 elements), so the
-    // unsigned 24-bit multiply is exact (a signed one would read snb >= 2^23 as negative);
-    // a chunk at or past the head dimension reads past the range (zeros), without a branch
-    const int off = (int)__umul24((unsigned)rowt, (unsigned)snb) + chunk * 16 + (chunk * 8 < a.D ? 0 : range);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst + wid_s * 1024), 16,
-                                             off, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int w4 = 2 * wid_s + j;
+      const int rowt = w4 * 4 + (lane >> 4);
+      const int pos = lane & 15;
+      const int chunk = pos ^ (isK ? (rowt & 15) : 4 * (rowt & 3));
+      // rowt < 32 and snb < 2^24 (the host limits sequence strides to 2^23 elements), so the
+      // unsigned 24-bit multiply is exact (a signed one would read snb >= 2^23 as negative);
+      // a chunk at or past the head dimension reads past the range (zeros), without a branch
+      const int off = (int)__umul24((unsigned)rowt, (unsigned)snb) + chunk * 16 + (chunk * 8 < a.D ? 0 : range);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst + w4 * 1024), 16,
+                                               off, 0, 0, 0);
+    }
   };
   // key biases (and timestamps) of the tile's 32 keys, into slot t % 4 of their ring
   // (lanes 32-63 read past the range: zeros); a packed tile reads the prepared biases,
@@ -813,11 +516,11 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   float mc[2] = {-__FLT_MAX__, -__FLT_MAX__}, l_i[2] = {0.0f, 0.0f};
   const float c = a.scale_log2;
 
-  unsigned stA = 0, stB = kWKBytes, stC = 2 * kWKBytes;
+  unsigned stA = 0, stB = kWKBytes;
   if (T > 0) {
     dma_rows(true, 0, stA);
     if (wid_s == 0) dma_meta(0);
-    dma_issue(1, 0, stB, stA);
+    dma_issue(1, 0, stB, stA);  // V of tile w - 1 is read in stage stB of window w
   }
   // ---- Q^T of both column blocks in registers, loaded while the first tiles are in
   // flight; rows past Nq load row Nq - 1 and dims past D dims 0..7, zeroed after ----
@@ -859,246 +562,214 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   constexpr int kWAhead = 3;    // V^T fragments read ahead of their MFMAs
   constexpr int kWQKAhead = 2;  // (K, Q) fragment pairs read ahead of their MFMAs
   const int nwin = T > 0 ? T + 1 : 0;
-  // One window = two sections.  Group 0 runs matrix(w), softmax(w); group 1 runs
-  // softmax(w - 1), matrix(w).  Each group has a loop of its own with the section kinds
-  // fixed at compile time, so that only P (group 0) or only S (group 1) is live across
-  // the loop's back edge.
-  auto section = [&](const int sec, auto GRP, auto ODD) {
-    constexpr int grp_c = decltype(GRP)::value;
-    constexpr bool odd = decltype(ODD)::value;
-    const int tl = sec >> 1;
-    const int sw = sec - grp_c;
-    // each wave issues its window's tile loads in its matrix section, after MFMA pair 6
-    bool issued = odd != (grp_c != 0);
-    auto issue_once = [&]() {
-      if (!issued) {
-        dma_issue(tl + 2, tl + 1, stC, stB);
-        issued = true;
+  // ---- matrix work of a window: O^T += V^T P^T for tile t - 1 (PV), then S^T = K Q^T for
+  // tile t (QK), each LDS fragment feeding both column blocks ----
+  // One stream of LDS operand reads for the section: the V^T fragments of the P.V
+  // block, then (hybrid, pure) the keys' biases, then the (K, Q) fragment pairs of
+  // the S^T block, each read a few MFMA pairs ahead of its use, across the border
+  // between the blocks.  The stream's order is fixed at compile time, so every wait
+  // is an exact lgkmcnt.
+  auto matrix_block = [&](const int t, auto PVC, auto QKC) __attribute__((always_inline)) {
+    constexpr bool PV = decltype(PVC)::value, QK = decltype(QKC)::value;
+    constexpr bool BIAS = QK && kWeights;
+    constexpr int NPV = PV ? 8 : 0, NQK = QK ? kD / 16 : 0;
+    constexpr int EBIAS = NPV;                   // stream index of the bias reads
+    constexpr int EQK = NPV + (BIAS ? 1 : 0);    // stream index of (K, Q) pair 0
+    constexpr int E = EQK + NQK;                 // stream length
+    constexpr int NM = NPV + NQK;                // MFMA pairs
+    // stream element of MFMA pair i; elements issued before pair i's wait
+    constexpr auto el = [](int i) { return i < NPV ? i : EQK + (i - NPV); };
+    constexpr auto size = [](int e) { return (BIAS && e == EBIAS) ? 4 : 2; };
+    constexpr auto issued = [el](int i) {
+      int n = 0;
+      for (int k = 0; k <= i; ++k) {
+        const int a = el(k) + 1 + (k < NPV ? kWAhead - 1 : kWQKAhead - 1);
+        n = a > n ? a : n;
+      }
+      return n < E ? n : E;
+    };
+    constexpr auto pending = [el, size, issued](int i) {
+      int c = 0;
+      for (int e = el(i) + 1; e < issued(i); ++e) c += size(e);
+      return c;
+    };
+    uint32_t va[4] = {0, 0, 0, 0};
+    if constexpr (PV) {
+      const uint32_t vb = lds_addr(vst0) + stB;
+      // opaque: otherwise the offsets are hoisted out of the loop into registers
+      asm volatile("" : "+v"(v_lane));
+      const uint32_t vl = vb + v_lane;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) va[db] = vl ^ (64u * db);
+    }
+    uint32_t kla = 0, qla = 0, bla = 0;
+    if constexpr (QK) {
+      asm volatile("" : "+v"(k_lane));
+      kla = lds_addr(kst0) + stA + k_lane;
+      qla = lds_addr(qs) + k_lane;
+      bla = lds_addr(meta_of(t) + kWCnt) + 16 * hl;
+    }
+    i16x4 vlo[8], vhi[8];
+    u32x4 kw[kD / 16], qw[kD / 16], bw[4];
+    auto read = [&](auto EC) {
+      constexpr int e = decltype(EC)::value;
+      if constexpr (e < NPV) {
+        vlo[e] = ds_read_tr16<(e >> 2) * 4096>(va[e & 3]);
+        vhi[e] = ds_read_tr16<(e >> 2) * 4096 + 2048>(va[e & 3]);
+      } else if constexpr (BIAS && e == EBIAS) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bw[r] = ds_read_b128_asm(bla + 32 * r);
+      } else {
+        constexpr int j = e - EQK;
+        kw[j] = ds_read_b128_asm(kla ^ (32u * j));
+        qw[j] = ds_read_b128_asm(qla ^ (32u * j));
       }
     };
-    if (sw >= 0) {
-      const int t = sw >> 1;
-      if constexpr (((odd ? 1 : 0) + grp_c) % 2 == 0) {
-        // ---- matrix section: O^T += V^T P^T for tile t-1, then S^T = K Q^T for tile t,
-        // each LDS fragment feeding both column blocks ----
-        __builtin_amdgcn_s_setprio(1);
-        const bool do_pv = t >= 1 && !skipped(t - 1);
-        const bool do_qk = t < T && !skipped(t);
-        // One stream of LDS operand reads for the section: the V^T fragments of the P.V
-        // block, then (hybrid, pure) the keys' biases, then the (K, Q) fragment pairs of
-        // the S^T block, each read a few MFMA pairs ahead of its use, across the border
-        // between the blocks.  The stream's order is fixed at compile time, so every wait
-        // is an exact lgkmcnt.
-        auto block = [&](auto PVC, auto QKC) {
-          constexpr bool PV = decltype(PVC)::value, QK = decltype(QKC)::value;
-          constexpr bool BIAS = QK && kWeights;
-          constexpr int NPV = PV ? 8 : 0, NQK = QK ? kD / 16 : 0;
-          constexpr int EBIAS = NPV;                   // stream index of the bias reads
-          constexpr int EQK = NPV + (BIAS ? 1 : 0);    // stream index of (K, Q) pair 0
-          constexpr int E = EQK + NQK;                 // stream length
-          constexpr int NM = NPV + NQK;                // MFMA pairs
-          // stream element of MFMA pair i; elements issued before pair i's wait
-          constexpr auto el = [](int i) { return i < NPV ? i : EQK + (i - NPV); };
-          constexpr auto size = [](int e) { return (BIAS && e == EBIAS) ? 4 : 2; };
-          constexpr auto issued = [el](int i) {
-            int n = 0;
-            for (int k = 0; k <= i; ++k) {
-              const int a = el(k) + 1 + (k < NPV ? kWAhead - 1 : kWQKAhead - 1);
-              n = a > n ? a : n;
-            }
-            return n < E ? n : E;
-          };
-          constexpr auto pending = [el, size, issued](int i) {
-            int c = 0;
-            for (int e = el(i) + 1; e < issued(i); ++e) c += size(e);
-            return c;
-          };
-          uint32_t va[4] = {0, 0, 0, 0};
-          if constexpr (PV) {
-            const uint32_t vb = lds_addr(vst0) + stC;
-            // opaque: otherwise the offsets are hoisted out of the loop into registers
-            asm volatile("" : "+v"(v_lane));
-            const uint32_t vl = vb + v_lane;
-#pragma unroll
-            for (int db = 0; db < 4; ++db) va[db] = vl ^ (64u * db);
-          }
-          uint32_t kla = 0, qla = 0, bla = 0;
-          if constexpr (QK) {
-            asm volatile("" : "+v"(k_lane));
-            kla = lds_addr(kst0) + stA + k_lane;
-            qla = lds_addr(qs) + k_lane;
-            bla = lds_addr(meta_of(t) + kWCnt) + 16 * hl;
-          }
-          i16x4 vlo[8], vhi[8];
-          u32x4 kw[kD / 16], qw[kD / 16], bw[4];
-          auto read = [&](auto EC) {
-            constexpr int e = decltype(EC)::value;
-            if constexpr (e < NPV) {
-              vlo[e] = ds_read_tr16<(e >> 2) * 4096>(va[e & 3]);
-              vhi[e] = ds_read_tr16<(e >> 2) * 4096 + 2048>(va[e & 3]);
-            } else if constexpr (BIAS && e == EBIAS) {
-#pragma unroll
-              for (int r = 0; r < 4; ++r) bw[r] = ds_read_b128_asm(bla + 32 * r);
-            } else {
-              constexpr int j = e - EQK;
-              kw[j] = ds_read_b128_asm(kla ^ (32u * j));
-              qw[j] = ds_read_b128_asm(qla ^ (32u * j));
-            }
-          };
-          static_for<issued(0)>(read);
-          static_for<NM>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            // the tile loads' scalar address work goes out between MFMA pairs 6 and 7,
-            // where it fills the matrix pipe's issue gaps (before pair 0 it delayed the
-            // first MFMA by about a hundred instructions)
-            if constexpr (i == 6) issue_once();
-            if constexpr (i < NPV) {
-              lgkm_wait<pending(i)>(vlo[i], vhi[i]);
-              const u32x4 vw = __builtin_bit_cast(u32x4, __builtin_shufflevector(vlo[i], vhi[i], 0, 1, 2, 3, 4, 5, 6, 7));
-              o[0][i & 3] = E16<DT>::mfma(vw, pw[0][i >> 2], o[0][i & 3]);
-              o[1][i & 3] = E16<DT>::mfma(vw, pw[1][i >> 2], o[1][i & 3]);
-            } else {
-              constexpr int j = i - NPV;
-              lgkm_wait<pending(i)>(kw[j], qw[j]);
-              if constexpr (j == 0) {
-                // S^T starts at the keys' biases (read before pair 0, so complete now),
-                // or at zero (the MFMA's inline constant)
-                if constexpr (BIAS) {
-                  asm volatile("" : "+v"(bw[0]), "+v"(bw[1]), "+v"(bw[2]), "+v"(bw[3]));
-                  const f32x4 b0 = __builtin_bit_cast(f32x4, bw[0]), b1 = __builtin_bit_cast(f32x4, bw[1]);
-                  const f32x4 b2 = __builtin_bit_cast(f32x4, bw[2]), b3 = __builtin_bit_cast(f32x4, bw[3]);
-                  const f32x16 c0 = __builtin_shufflevector(__builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                            __builtin_shufflevector(b2, b3, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                            0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-                  s[0] = E16<DT>::mfma(kw[0], qreg[0], c0);
-                  s[1] = E16<DT>::mfma(kw[0], qw[0], c0);
-                } else {
-                  s[0] = E16<DT>::mfma(kw[0], qreg[0], f32x16{});
-                  s[1] = E16<DT>::mfma(kw[0], qw[0], f32x16{});
-                }
-              } else {
-                s[0] = E16<DT>::mfma(kw[j], qreg[j], s[0]);
-                s[1] = E16<DT>::mfma(kw[j], qw[j], s[1]);
-              }
-            }
-            static_for<issued(i + 1 < NM ? i + 1 : i) - issued(i)>([&](auto K) {
-              read(std::integral_constant<int, issued(i) + decltype(K)::value>{});
-            });
-          });
-        };
-        using BT = std::integral_constant<bool, true>;
-        using BF = std::integral_constant<bool, false>;
-        // The S^T block always runs: where tile t is past the end or skipped, it reads a
-        // stage and a bias slot that hold other data (in bounds) and the softmax ignores
-        // the result.  A third instantiation without it costs more registers than the
-        // few blocks it saves.
-        if (do_pv)
-          block(BT{}, BT{});
-        else
-          block(BF{}, BT{});
-        issue_once();
-        if (!do_qk) {
-          // not read before the next QK block defines it
-          undefined(s[0]);
-          undefined(s[1]);
-        }
-        __builtin_amdgcn_s_setprio(0);
-      } else if (!(t < T && !skipped(t))) {
-        // not read before the next softmax defines it
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) undefined(pw[cb][j]);
+    static_for<issued(0)>(read);
+    static_for<NM>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i < NPV) {
+        lgkm_wait<pending(i)>(vlo[i], vhi[i]);
+        const u32x4 vw = __builtin_bit_cast(u32x4, __builtin_shufflevector(vlo[i], vhi[i], 0, 1, 2, 3, 4, 5, 6, 7));
+        o[0][i & 3] = E16<DT>::mfma(vw, pw[0][i >> 2], o[0][i & 3]);
+        o[1][i & 3] = E16<DT>::mfma(vw, pw[1][i >> 2], o[1][i & 3]);
       } else {
-        // ---- softmax section for tile t: the two column blocks one after the other, one
-        // check each ----
-        const char* ms = meta_of(t);
-        const int key0 = key0_of(t);
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          const int row = r0w + 32 * cb + ql;
-          if (kPureV) {
-            mask_pure32(s[cb], (const int*)(ms + kWTs), row, hl);
-          } else if (t >= n1) {
-            if ((a.causal && key0 + kWTK - 1 > r0w + 32 * cb) || key0 + kWTK > Nk)
-              mask_dense32(s[cb], key0, row, hl, Nk, a.causal);
+        constexpr int j = i - NPV;
+        lgkm_wait<pending(i)>(kw[j], qw[j]);
+        if constexpr (j == 0) {
+          // S^T starts at the keys' biases (read before pair 0, so complete now),
+          // or at zero (the MFMA's inline constant)
+          if constexpr (BIAS) {
+            asm volatile("" : "+v"(bw[0]), "+v"(bw[1]), "+v"(bw[2]), "+v"(bw[3]));
+            const f32x4 b0 = __builtin_bit_cast(f32x4, bw[0]), b1 = __builtin_bit_cast(f32x4, bw[1]);
+            const f32x4 b2 = __builtin_bit_cast(f32x4, bw[2]), b3 = __builtin_bit_cast(f32x4, bw[3]);
+            const f32x16 c0 = __builtin_shufflevector(__builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7),
+                                                      __builtin_shufflevector(b2, b3, 0, 1, 2, 3, 4, 5, 6, 7),
+                                                      0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+            s[0] = E16<DT>::mfma(kw[0], qreg[0], c0);
+            s[1] = E16<DT>::mfma(kw[0], qw[0], c0);
+          } else {
+            s[0] = E16<DT>::mfma(kw[0], qreg[0], f32x16{});
+            s[1] = E16<DT>::mfma(kw[0], qw[0], f32x16{});
           }
-        }
-        // p against the current maximum first; only where a lane's sum of its 16 p
-        // exceeds kLazySum (some p above 2^8, a score above the maximum by 8 / c; +inf
-        // while the lane has no maximum yet) is the tile's maximum taken and the column
-        // block redone with the lazy-rescale rule.  P in the 16-bit type for the P.V
-        // MFMAs; the row sum adds the fp32 p, as deltaFlashAttention.py:86-98
-        auto exps = [&](const int cb, const float neg) {
-          float psa, psb;
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            float p[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) p[e] = exp2_fast(__builtin_fmaf(s[cb][4 * r4 + e], c, neg));
-            pw[cb][r4 >> 1][(r4 & 1) * 2 + 0] = E16<DT>::pack(p[0], p[1]);
-            pw[cb][r4 >> 1][(r4 & 1) * 2 + 1] = E16<DT>::pack(p[2], p[3]);
-            psa = r4 == 0 ? p[0] + p[1] : psa + (p[0] + p[1]);
-            psb = r4 == 0 ? p[2] + p[3] : psb + (p[2] + p[3]);
-          }
-          return psa + psb;
-        };
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          float ps = exps(cb, -mc[cb]);
-          // the bound also catches an infinite sum
-          if (__builtin_amdgcn_ballot_w64(ps > kLazySum)) {
-            float m = -INFINITY;
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) m = __builtin_fmaxf(m, __builtin_fmaxf(s[cb][r], s[cb][r + 1]));
-            const float mxc = halves_max(m) * c;
-            // alpha = 1 exactly where a lane keeps its maximum (also where it has none yet)
-            const bool upd = mxc > mc[cb] + kLazyLog2;
-            const float m_new = upd ? mxc : mc[cb];
-            const float alpha = upd ? exp2_fast(mc[cb] - m_new) : 1.0f;
-#pragma unroll
-            for (int db = 0; db < 4; ++db)
-#pragma unroll
-              for (int r = 0; r < 16; ++r) o[cb][db][r] *= alpha;
-            l_i[cb] *= alpha;
-            mc[cb] = m_new;
-            ps = exps(cb, -m_new);
-          }
-          l_i[cb] += ps;
+        } else {
+          s[0] = E16<DT>::mfma(kw[j], qreg[j], s[0]);
+          s[1] = E16<DT>::mfma(kw[j], qw[j], s[1]);
         }
       }
+      static_for<issued(i + 1 < NM ? i + 1 : i) - issued(i)>([&](auto K) {
+        read(std::integral_constant<int, issued(i) + decltype(K)::value>{});
+      });
+    });
+  };
+  // ---- softmax of tile t: the two column blocks one after the other, one check each ----
+  auto softmax_tile = [&](const int t) __attribute__((always_inline)) {
+    const char* ms = meta_of(t);
+    const int key0 = key0_of(t);
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      const int row = r0w + 32 * cb + ql;
+      if (kPureV) {
+        mask_pure32(s[cb], (const int*)(ms + kWTs), row, hl);
+      } else if (t >= n1) {
+        if ((a.causal && key0 + kWTK - 1 > r0w + 32 * cb) || key0 + kWTK > Nk)
+          mask_dense32(s[cb], key0, row, hl, Nk, a.causal);
+      }
     }
-    issue_once();
-    if (odd) {
-      // the loads of window tl - 1 are done when at most this window's are pending
-      if (wid_s == 0)
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(2 + (kWeights ? 1 : 0) + (kPureV ? 1 : 0)));
-      else
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(2));
-      barrier_keep_loads();
+    // p against the current maximum first; only where a lane's sum of its 16 p
+    // exceeds kLazySum (some p above 2^8, a score above the maximum by 8 / c; +inf
+    // while the lane has no maximum yet) is the tile's maximum taken and the column
+    // block redone with the lazy-rescale rule.  P in the 16-bit type for the P.V
+    // MFMAs; the row sum adds the fp32 p, as deltaFlashAttention.py:86-98
+    auto exps = [&](const int cb, const float neg) {
+      float psa, psb;
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        float p[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[e] = exp2_fast(__builtin_fmaf(s[cb][4 * r4 + e], c, neg));
+        pw[cb][r4 >> 1][(r4 & 1) * 2 + 0] = E16<DT>::pack(p[0], p[1]);
+        pw[cb][r4 >> 1][(r4 & 1) * 2 + 1] = E16<DT>::pack(p[2], p[3]);
+        psa = r4 == 0 ? p[0] + p[1] : psa + (p[0] + p[1]);
+        psb = r4 == 0 ? p[2] + p[3] : psb + (p[2] + p[3]);
+      }
+      return psa + psb;
+    };
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      float ps = exps(cb, -mc[cb]);
+      // the bound also catches an infinite sum
+      if (__builtin_amdgcn_ballot_w64(ps > kLazySum)) {
+        float m = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) m = __builtin_fmaxf(m, __builtin_fmaxf(s[cb][r], s[cb][r + 1]));
+        const float mxc = halves_max(m) * c;
+        // alpha = 1 exactly where a lane keeps its maximum (also where it has none yet)
+        const bool upd = mxc > mc[cb] + kLazyLog2;
+        const float m_new = upd ? mxc : mc[cb];
+        const float alpha = upd ? exp2_fast(mc[cb] - m_new) : 1.0f;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[cb][db][r] *= alpha;
+        l_i[cb] *= alpha;
+        mc[cb] = m_new;
+        ps = exps(cb, -m_new);
+      }
+      l_i[cb] += ps;
     }
   };
   using False = std::integral_constant<bool, false>;
   using True = std::integral_constant<bool, true>;
-  auto rotate_stages = [&]() {
+  // Window w: the matrix work, the barrier, the loads of the next windows, the softmax.
+  // At the barrier every wave has read K of tile w and V of tile w - 1, and the loads of
+  // window w - 1 (K of w + 1, V of w) are done: K of w + 2 and V of w + 1 take their stages.
+  auto turn = [&](const int w) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    barrier_keep_loads();
+    if (w < T) dma_issue(w + 2, w + 1, stA, stB);
+  };
+  auto swap_stages = [&]() {
     const unsigned t0 = stA;
     stA = stB;
-    stB = stC;
-    stC = t0;
+    stB = t0;
   };
-  if (grp == 0) {
-    for (int w = 0; w < nwin; ++w) {
-      section(2 * w, std::integral_constant<int, 0>{}, False{});
-      section(2 * w + 1, std::integral_constant<int, 0>{}, True{});
-      rotate_stages();
+  int w = 0;
+  auto idle_until = [&](const int end) {  // windows whose tiles are not the wave's
+    for (; w < end; ++w) {
+      turn(w);
+      swap_stages();
     }
-  } else {
-    for (int w = 0; w < nwin; ++w) {
-      section(2 * w, std::integral_constant<int, 1>{}, False{});
-      section(2 * w + 1, std::integral_constant<int, 1>{}, True{});
-      rotate_stages();
+  };
+  // The wave's tiles are one interval, or two around the other logical block's.  Each runs
+  // a loop without conditions (with them, its registers do not fit).
+  const bool gap = skip_lo < skip_hi;
+#pragma nounroll
+  for (int r = 0; r < 2; ++r) {
+    const int lo = r ? skip_hi : 0;
+    const int hi = min(min(T, t_skip), r ? (gap ? T : 0) : (gap ? skip_lo : T));
+    if (lo >= hi) continue;
+    idle_until(lo);
+    __builtin_amdgcn_s_setprio(1);
+    matrix_block(w, False{}, True{});
+    __builtin_amdgcn_s_setprio(0);
+    turn(w);
+    softmax_tile(w);
+    swap_stages();
+    for (++w; w < hi; ++w) {
+      __builtin_amdgcn_s_setprio(1);
+      matrix_block(w, True{}, True{});
+      __builtin_amdgcn_s_setprio(0);
+      turn(w);
+      softmax_tile(w);
+      swap_stages();
     }
+    matrix_block(w, True{}, False{});
+    turn(w);
+    swap_stages();
+    ++w;
   }
+  idle_until(nwin);
   __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // no load may land in LDS after the exit
 
   // ---- finalize: each column block goes through the wave's own Q region of LDS (its
@@ -1149,15 +820,15 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
 // i mod 8 and takes one item; when the units split evenly over the 8 XCDs, each XCD gets
 // a contiguous range of units and walks their row groups longest first, so a unit's K/V
 // stay in one XCD's L2.  Persistent (a.queue set, the hybrid, sanity and pure Phase 1
-// variants, whose schedule kernel zeroes the 8 counters just before): one workgroup per
-// CU loops over items.  Queue q holds the units of XCD q's static share in the same
+// variants, whose schedule kernel zeroes the 8 counters just before): two workgroups per
+// CU loop over items.  Queue q holds the units of XCD q's static share in the same
 // order (unit by unit, longest row group first) and a.queue[q] counts the items taken;
 // a workgroup takes from the queue of the XCD it runs on and, once that is empty, from
 // the others, so the XCDs, whose clocks differ by several per cent, finish together,
 // and no dispatch gap lies between two items on a CU.  Every counter only grows, so each
 // workgroup's loop ends after at most 8 empty takes; workgroups never wait on each other.
 template <int VARIANT, int DT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_w64_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int* const slot = (int*)(smem + kWItemSlot);
@@ -1175,9 +846,11 @@ void attn_w64_kernel(AttnArgs a) {
       if (!first) break;
       const int wg = blockIdx.x;
       if ((a.units & 7) == 0) {
-        const int xcd = wg & 7, idx = wg >> 3, upx = a.units >> 3;
-        unit = xcd * upx + idx / n_rg;
-        rg = n_rg - 1 - idx % n_rg;
+        const int xcd = wg & 7, upx = a.units >> 3;
+        item_at(wg >> 3, upx, n_rg, a.slots, unit, rg);
+        unit += xcd * upx;
+      } else if (a.units * n_rg <= 8 * a.slots) {
+        item_at(wg, a.units, n_rg, 8 * a.slots, unit, rg);
       } else {
         unit = wg % a.units;
         rg = n_rg - 1 - wg / a.units;
@@ -1207,9 +880,8 @@ void attn_w64_kernel(AttnArgs a) {
       if (k < 0) break;
       int ulo, uhi;
       queue_units(q, a.units, ulo, uhi);
-      const int j = k / n_rg;
-      unit = ulo + j;
-      rg = n_rg - 1 - (k - j * n_rg);
+      item_at(k, uhi - ulo, n_rg, a.slots, unit, rg);
+      unit += ulo;
     }
 #if defined(__HIP_DEVICE_COMPILE__)
     // the argument block read through the kernel-argument segment's address, made
@@ -1228,7 +900,9 @@ void attn_w64_kernel(AttnArgs a) {
 }
 
 // Per (batch, kv head): maxima of packed blocks of 128 timestamps (lanes at or
-// beyond P read seq_len_k + 1, deltaFlashAttention.py:70) and their prefix maxima.
+// beyond P read seq_len_k + 1, deltaFlashAttention.py:70) and their prefix maxima; for pure
+// Phase 1 the suffix minima instead, which end a row group's keys at the last block that
+// holds one it sees (16384 tokens, one key in four: 587 against 1018 us).
 // Blocks with blockIdx.y = 0 do that; those with blockIdx.y = 1 + c (when wts is set)
 // write, for packed rows [1024 c, 1024 c + 1024), the key bias log2(w) / scale_log2 of
 // the row's weight w (the count, 1 with no_count, 0 at and beyond P:
@@ -1275,7 +949,7 @@ __global__ __launch_bounds__(kSchedThreads) void hybrid_schedule_kernel(const in
     const int32_t* crow = (const int32_t*)prep.cnt + seq.base(b, prep.scnt_b, 1) + (int64_t)g * prep.scnt_h;
     float* wrow = prep.wts + (int64_t)bg * prep.wcap;
     int32_t* trow = prep.tsw ? prep.tsw + (int64_t)bg * prep.wcap : nullptr;
-    if (bg == 0 && blockIdx.y == 1 && tid < kTileN) prep.zeros[tid] = 0.0f;
+    if (bg == 0 && blockIdx.y == 1 && tid < 64) prep.zeros[tid] = 0.0f;
     // the attention kernels read rows below nblk * 128 only
     const int i = (blockIdx.y - 1) * kSchedThreads + tid;
     if ((blockIdx.y - 1) * kSchedThreads >= nblk * kBlock || i >= prep.wcap) return;
@@ -1290,6 +964,12 @@ __global__ __launch_bounds__(kSchedThreads) void hybrid_schedule_kernel(const in
     if (trow) trow[i] = tv;
     return;
   }
+  // Pure Phase 1 takes all packed keys, masked by timestamp <= row: its rows need the blocks
+  // up to the last one that holds such a key, so the scan is of the blocks' minima (keys of
+  // weight 0 left out), from the last block back, as maxima of the negated values.
+  const bool pure = prep.tsw != nullptr;
+  const int32_t* crow = pure ? (const int32_t*)prep.cnt + seq.base(b, prep.scnt_b, 1) + (int64_t)g * prep.scnt_h : row;
+  auto weighs = [&](int32_t raw) { return prep.no_count || (prep.cnt_is_float ? __int_as_float(raw) > 0.0f : raw > 0); };
   // wave w takes blocks 8w .. 8w + 7 of every 8 kSchedWaves, their loads in flight together:
   // rows at or beyond P are clamped to row P - 1 and masked after the load (a guarded
   // load is waited for before the next one is issued); nblk > 0 implies P > 0
@@ -1302,16 +982,31 @@ __global__ __launch_bounds__(kSchedThreads) void hybrid_schedule_kernel(const in
       r0[u] = row[min(i0, P - 1)];
       r1[u] = row[min(i1, P - 1)];
     }
+    if (pure) {
+      int c0[8], c1[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i0 = (jb0 + u) * kBlock + lane, i1 = i0 + 64;
-      m[u] = max(i0 < P ? r0[u] : Nk + 1, i1 < P ? r1[u] : Nk + 1);
+      for (int u = 0; u < 8; ++u) {
+        const int i0 = (jb0 + u) * kBlock + lane, i1 = i0 + 64;
+        c0[u] = crow[min(i0, P - 1)];
+        c1[u] = crow[min(i1, P - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i0 = (jb0 + u) * kBlock + lane, i1 = i0 + 64;
+        m[u] = max(i0 < P && weighs(c0[u]) ? -r0[u] : -INT_MAX, i1 < P && weighs(c1[u]) ? -r1[u] : -INT_MAX);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i0 = (jb0 + u) * kBlock + lane, i1 = i0 + 64;
+        m[u] = max(i0 < P ? r0[u] : Nk + 1, i1 < P ? r1[u] : Nk + 1);
+      }
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
 #pragma unroll
       for (int d = 32; d >= 1; d >>= 1) m[u] = max(m[u], __shfl_xor(m[u], d, 64));
-      if (lane == 0 && jb0 + u < nblk) s_bmax[jb0 + u] = m[u];
+      if (lane == 0 && jb0 + u < nblk) s_bmax[pure ? nblk - 1 - (jb0 + u) : jb0 + u] = m[u];
     }
   }
   __syncthreads();
@@ -1336,8 +1031,12 @@ __global__ __launch_bounds__(kSchedThreads) void hybrid_schedule_kernel(const in
   int32_t* pm = bm + nblk_cap;
   for (int j = j0; j < j1; ++j) {
     run = max(run, s_bmax[j]);
-    bm[j] = s_bmax[j];
-    pm[j] = run;
+    if (pure) {
+      pm[nblk - 1 - j] = -run;  // the least timestamp from block nblk - 1 - j on
+    } else {
+      bm[j] = s_bmax[j];
+      pm[j] = run;
+    }
   }
 }
 
@@ -1447,7 +1146,11 @@ void attn_f32_kernel(AttnArgs a, int paired) {
     ds = max(0, ((last + 1) / kBlock) * kBlock);
     if (VARIANT == kHybrid) n1 = min(n_safe * kBlock, a.wcap);
   } else if (VARIANT == kPure) {
-    n1 = P;
+    // the packed blocks up to the last that holds a key at or before the last row
+    const int32_t* from = a.sched + (int64_t)bg * 2 * a.nblk_cap + a.nblk_cap;
+    int last;
+    safe_prefix(from, from, (P + kBlock - 1) / kBlock, R0 + kFRows, n1, last, lane);
+    n1 = min(n1 * kBlock, P);
     kend = 0;
   }
   const int t1 = (n1 + kFTile - 1) / kFTile;
@@ -1621,24 +1324,6 @@ void attn_f32_kernel(AttnArgs a, int paired) {
     if (d0 + i < D) *(f32x2*)(orow + d0 + i) = f32x2{x[i], x[i + 1]};
 }
 
-template <int V, int DT>
-static const void* attn_kernel_fn() {
-  if constexpr (V == kPure) return reinterpret_cast<const void*>(&attn_kernel_pure<DT>);
-  else return reinterpret_cast<const void*>(&attn_kernel<V, DT>);
-}
-
-template <int V, int DT>
-static int allow_lds(size_t bytes) {
-  static int done = 0;
-  if (!done) {
-    hipError_t e = hipFuncSetAttribute(attn_kernel_fn<V, DT>(),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e != hipSuccess) return set_error(DA_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-    done = 1;
-  }
-  return DA_OK;
-}
-
 // Compute units of the current device (cached per device).
 static int cu_count() {
   static int n[64] = {};
@@ -1653,38 +1338,20 @@ static int cu_count() {
 }
 
 template <int V, int DT>
-static int allow_lds_w64(size_t bytes) {
+static int launch_attn_t(AttnArgs& a, hipStream_t st) {
   static int done = 0;
   if (!done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_w64_kernel<V, DT>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kWLds);
     if (e != hipSuccess) return set_error(DA_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     done = 1;
   }
-  return DA_OK;
-}
-
-template <int V, int DT>
-static int launch_attn_t(AttnArgs& a, hipStream_t st) {
-  if (a.hpw == 4) {
-    a.rows_per_wg = 128;
-    a.n_row_groups = (a.Nq + 127) / 128;
-    const size_t lds = kWLds;
-    const int64_t items = (int64_t)a.n_row_groups * a.units;
-    // persistent: one workgroup per CU (the LDS of one fills a CU) takes items until the
-    // queues are empty; static: one workgroup per item
-    const unsigned grid = (unsigned)(a.queue ? std::min<int64_t>(items, cu_count()) : items);
-    if (int rc = allow_lds_w64<V, DT>(lds)) return rc;
-    hipLaunchKernelGGL((attn_w64_kernel<V, DT>), dim3(grid), dim3(512), lds, st, a);
-    return check_launch("attention kernel (ping-pong)");
-  }
-  const size_t lds = 2 * kStageBytes;
-  const unsigned grid = (unsigned)((int64_t)a.n_row_groups * a.units);
-  if (int rc = allow_lds<V, DT>(lds)) return rc;
-  if constexpr (V == kPure)
-    hipLaunchKernelGGL((attn_kernel_pure<DT>), dim3(grid), dim3(256), lds, st, a);
-  else
-    hipLaunchKernelGGL((attn_kernel<V, DT>), dim3(grid), dim3(256), lds, st, a);
+  a.slots = 2 * cu_count() / 8;
+  const int64_t items = (int64_t)a.n_row_groups * a.units;
+  // persistent: as many workgroups as run at once (two a CU) take items until the queues are
+  // empty; static: one workgroup per item
+  const unsigned grid = (unsigned)(a.queue ? std::min<int64_t>(items, 2 * cu_count()) : items);
+  hipLaunchKernelGGL((attn_w64_kernel<V, DT>), dim3(grid), dim3(256), kWLds, st, a);
   return check_launch("attention kernel");
 }
 
@@ -1758,7 +1425,7 @@ static int fill_common(AttnArgs& a, const void* q, const void* k, const void* v,
   a.D = (int)D;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.hpw = (a.G % 4 == 0) ? 4 : (a.G % 2 == 0 ? 2 : 1);
-  a.rows_per_wg = 32 * (4 / a.hpw);
+  a.rows_per_wg = 256 / a.hpw;
   a.n_row_groups = (int)((Nq + a.rows_per_wg - 1) / a.rows_per_wg);
   a.units = (int)(B * Hkv * (a.G / a.hpw));
   DA_REQUIRE((int64_t)a.n_row_groups * a.units < (1ll << 31), "%s: grid too large", who);
@@ -1855,8 +1522,8 @@ static int hybrid_impl(const char* who, AttnArgs& a, const void* k_packed, const
     prep.wcap = wl.wcap;
   }
   const unsigned prep_chunks = prep.wts ? (unsigned)((wl.wcap + kSchedThreads - 1) / kSchedThreads) : 0u;
-  // the grouped kernel's persistent grid takes its items from 8 counters in the workspace
-  a.queue = a.hpw == 4 && dtype != DA_F32 ? (int*)(ws + wl.queue_off) : nullptr;
+  // the 16-bit kernel's persistent grid takes its items from 8 counters in the workspace
+  a.queue = dtype != DA_F32 ? (int*)(ws + wl.queue_off) : nullptr;
   hipLaunchKernelGGL(hybrid_schedule_kernel, dim3((unsigned)(B * Hkv), 1 + prep_chunks), dim3(kSchedThreads), 0, st,
                      timestamps, a.sts_b, a.sts_h, (int)Hkv, (int)P_bound, num_packed_dev, (int)Nk, a.seq,
                      a.nblk_cap, (int32_t*)ws, prep, a.queue);

@@ -1,0 +1,73 @@
+"""The 16-bit attention kernel at the edges of its items (64, 128 and 256 rows), tiles and
+grids, for every kind of GQA group, against the oracle (fp32 on the same 16-bit inputs).
+
+Tolerance: the bars every bf16 / fp16 attention output of this build is held to (max-abs
+2e-2, mean-abs 1e-3): P is rounded to the 16-bit type before P.V and the output is stored in
+it, 2^-9 of values below 4 each.
+"""
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce, oracle_arith
+from oracle import delta_oracle as O
+from oracle import select_oracle_c as OC
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(out, want):
+    err = np.abs(out.float().cpu().numpy() - want)
+    assert err.max() <= 2e-2 and err.mean() <= 1e-3, (err.max(), err.mean())
+
+
+@pytest.mark.parametrize("variant", ["hybrid", "sanity", "pure_phase1"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,W,chunk", [
+    (1, 3, 3, 255, 64, 0, 64), (1, 2, 2, 257, 128, 64, 64), (1, 2, 1, 385, 128, 128, 100),
+    (2, 6, 2, 640, 72, 0, 32), (1, 8, 1, 65, 128, 64, 512), (1, 12, 3, 193, 128, 0, 64),
+    (1, 4, 4, 1400, 128, 128, 128), (1, 5, 1, 900, 8, 64, 128)])
+def test_groups_and_row_edges(gpu, variant, B, Hq, Hkv, N, D, W, chunk):
+    """One head over two logical blocks (their schedules differ), two heads over one, four
+    over half of one; the last item partly or wholly past the rows."""
+    from deltaattention_amd import ops, synth
+    q, k, v = synth.make_layer_inputs(B, Hq, Hkv, N, D, seed=N + D)
+    tau = 9.0 * (D / 128) ** 0.5
+    announce(f"attn edges {variant} B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} W={W}")
+    out = ops.delta_prefill(q.to(gpu), k.to(gpu), v.to(gpu), tau, chunk, window=W, variant=variant)
+    kf, vf = k.float().numpy(), v.float().numpy()
+    keep, _ = OC.select_delta(kf, tau, chunk, arith=oracle_arith(k))
+    p = O.pack(kf, vf, keep)
+    _close(out, O.hybrid_attention(q.float().numpy(), kf, vf, p["k_packed"], p["v_packed"], p["timestamps"],
+                                   p["counts"], W, variant=variant))
+
+
+@pytest.mark.parametrize("Hq,Hkv,N,causal", [
+    (1, 1, 1, True), (7, 7, 63, True), (2, 2, 256, False), (6, 3, 129, True), (32, 8, 1056, True),
+    (16, 16, 513, True), (40, 8, 300, False), (64, 16, 600, True)])
+def test_dense_small_grids(gpu, Hq, Hkv, N, causal):
+    """Grids of less than one, between one and two, and more workgroups than run at once."""
+    from deltaattention_amd import ops, synth
+    q, k, v = synth.make_layer_inputs(1, Hq, Hkv, N, 128, seed=N)
+    announce(f"dense Hq={Hq} Hkv={Hkv} N={N} causal={causal}")
+    out = ops.dense_prefill(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal)
+    _close(out, O.dense_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), causal))
+
+
+def test_pure_phase1_unsorted_timestamps(gpu):
+    """Pure Phase 1 ends a row group's keys at the last packed block that holds a timestamp it
+    sees: with the packed rows in a random order, and some of weight 0, that is the bound the
+    suffix minima give, and the result the oracle's."""
+    from deltaattention_amd import ops, synth
+    N, P = 1000, 300
+    q, k, v = synth.make_layer_inputs(1, 4, 2, N, 128, seed=3)
+    rng = np.random.default_rng(0)
+    ts = np.stack([1 + rng.permutation(N - 1)[:P] for _ in range(2)])[None].astype(np.int32)
+    cnt = rng.integers(0, 4, size=ts.shape).astype(np.int32)
+    ts[..., 5], cnt[..., 5] = 0, 2  # every row sees a key in the first block
+    kp = torch.stack([k[0, h, torch.from_numpy(ts[0, h]).long()] for h in range(2)])[None].contiguous()
+    vp = torch.stack([v[0, h, torch.from_numpy(ts[0, h]).long()] for h in range(2)])[None].contiguous()
+    announce("pure phase 1, unsorted timestamps")
+    out = ops.hybrid_prefill(q.to(gpu), k.to(gpu), v.to(gpu), kp.to(gpu), vp.to(gpu), torch.from_numpy(ts).to(gpu),
+                             torch.from_numpy(cnt).to(gpu), window=64, variant="pure_phase1")
+    _close(out, O.hybrid_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), kp.float().numpy(),
+                                   vp.float().numpy(), ts, cnt, 64, variant="pure_phase1"))
