@@ -9,6 +9,8 @@ import ctypes
 import os
 import threading
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libdeltaattn.so")
 
@@ -119,22 +121,42 @@ def check(rc: int, what: str) -> None:
         raise DeltaAttnError(what, rc, msg.decode() if msg else "")
 
 
+_Strides = ctypes.c_int64 * DA_NUM_STRIDES
+
+
 def strides_array(values) -> ctypes.Array:
-    arr = (ctypes.c_int64 * DA_NUM_STRIDES)()
-    for i, v in enumerate(values):
-        arr[i] = int(v)
-    return arr
+    return _Strides(*values)
+
+
+_CODES = {torch.bfloat16: DA_BF16, torch.float16: DA_F16, torch.float32: DA_F32}
 
 
 def dtype_code(*ts) -> int:
     """DA_BF16, DA_F16 or DA_F32 for tensors that all share one of those dtypes (the entry
     points that do not take fp32, the decode ones, refuse DA_F32 with DA_ERR_UNSUPPORTED)."""
-    import torch
-    codes = {torch.bfloat16: DA_BF16, torch.float16: DA_F16, torch.float32: DA_F32}
     dt = ts[0].dtype
-    if dt not in codes:
+    code = _CODES.get(dt)
+    if code is None:
         raise TypeError(f"expected bfloat16, float16 or float32 tensors, got {dt}")
     for t in ts[1:]:
         if t is not None and t.dtype != dt:
             raise TypeError(f"all tensors must share one dtype ({dt}), got {t.dtype}")
-    return codes[dt]
+    return code
+
+
+def current_stream() -> int:
+    """The handle of the current device's current stream, without building a torch Stream
+    object."""
+    return _raw_stream(torch.cuda.current_device())
+
+
+def device_stream(device: torch.device) -> int:
+    """The handle of the current stream of ``device``."""
+    return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
+
+
+def _raw_stream(index: int) -> int:
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if get is None:  # pragma: no cover - older torch
+        return torch.cuda.current_stream(index).cuda_stream
+    return get(index)

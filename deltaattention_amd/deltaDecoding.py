@@ -16,7 +16,7 @@ import torch
 
 from . import globVR
 from ._launch import HALF, KernelLauncher, tensor, unit_stride
-from ._native import DecodeStep, check, dtype_code, lib
+from ._native import DecodeStep, check, current_stream, device_stream, dtype_code, lib
 
 try:  # transformers' Cache base (the reference subclasses it, deltaDecoding.py:2, 111)
     from transformers import Cache as _CacheBase
@@ -28,15 +28,7 @@ __all__ = ["HybridCompressedCache", "fused_hybrid_decode_update_kernel",
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
-def _raw_stream(device: torch.device) -> int:
-    """The current stream's handle without building a torch Stream object."""
-    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if get is None:  # pragma: no cover - older torch
-        return torch.cuda.current_stream(device).cuda_stream
-    return get(device.index if device.index is not None else torch.cuda.current_device())
+    return ctypes.c_void_p(current_stream())
 
 
 def _metric_threshold():
@@ -282,7 +274,7 @@ class HybridCompressedCache(_CacheBase):
         ws_bytes = lib().da_decode_workspace_size(self.bsz, Hq, self.capacity, self.exact_window_size)
         ws = torch.empty((max(1, ws_bytes),), dtype=torch.uint8, device=self.device)
         st.workspace, st.workspace_bytes = ws.data_ptr(), ws_bytes
-        plan = (st, ws, ctypes.byref(st))
+        plan = (st, ws, ctypes.byref(st), kp.dtype)
         self._plans[key] = plan
         return plan
 
@@ -296,41 +288,42 @@ class HybridCompressedCache(_CacheBase):
         another order (the new anchor is scored at the end of its key list)."""
         if self.max_packed_len[layer_idx] + 1 >= self.capacity:
             self._expand_capacity(self.capacity + 1024)
-        B, Hq, _, D = query_states.shape
+        B, Hq, n, D = query_states.shape
         want = (self.bsz, self.n_kv_heads, 1, self.head_dim)
-        if (B, D) != (self.bsz, self.head_dim) or query_states.shape[2] != 1 \
-                or tuple(key_states.shape) != want or tuple(value_states.shape) != want:
+        if n != 1 or B != self.bsz or D != self.head_dim or key_states.shape != want \
+                or value_states.shape != want:
             raise ValueError(f"decode_step: expected q [{self.bsz}, Hq, 1, {self.head_dim}] and "
                              f"key/value {list(want)}, got {list(query_states.shape)}, "
                              f"{list(key_states.shape)}, {list(value_states.shape)}")
-        st, ws, ref = self._plan(layer_idx, Hq)
-        q = query_states.squeeze(2)
-        if q.stride(-1) != 1:
-            q = q.contiguous()
-        k = key_states if key_states.stride(-1) == 1 else key_states.contiguous()
-        v = value_states if value_states.stride(-1) == 1 else value_states.contiguous()
-        if k.stride()[:2] != v.stride()[:2]:
-            k, v = k.contiguous(), v.contiguous()
-        if dtype_code(q, k, v) != st.dtype:
+        st, ws, ref, dtype = self._plan(layer_idx, Hq)
+        q, k, v = query_states, key_states, value_states
+        if not q.dtype == k.dtype == v.dtype == dtype:
             raise TypeError("decode_step: query, key and value must have the cache's dtype")
-        out = torch.empty((B, Hq, D), dtype=q.dtype, device=q.device)
+        sq, sk, sv = q.stride(), k.stride(), v.stride()
+        if sq[3] != 1:
+            q = q.contiguous()
+            sq = q.stride()
+        if sk[3] != 1 or sv[3] != 1 or sk[0] != sv[0] or sk[1] != sv[1]:
+            k, v = k.contiguous(), v.contiguous()
+            sk = k.stride()
+        out = torch.empty((B, Hq, 1, D), dtype=dtype, device=q.device)
         threshold, use_cos = _metric_threshold()
-        st.new_k, st.new_v, st.sn_b, st.sn_h = k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1)
-        st.q, st.sq_b, st.sq_h = q.data_ptr(), q.stride(0), q.stride(1)
-        st.out, st.so_b, st.so_h = out.data_ptr(), out.stride(0), out.stride(1)
+        st.new_k, st.new_v, st.sn_b, st.sn_h = k.data_ptr(), v.data_ptr(), sk[0], sk[1]
+        st.q, st.sq_b, st.sq_h = q.data_ptr(), sq[0], sq[1]
+        st.out, st.so_b, st.so_h = out.data_ptr(), Hq * D, D
         st.exact_seq_len = self.exact_seq_lens[layer_idx]
         st.total_seq_len = self.total_seq_lens[layer_idx]
         st.threshold = float(threshold)
         st.use_cosine = 1 if use_cos else 0
         st.scale = D ** -0.5 if scaling is None else float(scaling)
-        check(lib().da_decode_step(ref, _raw_stream(q.device)), "HybridCompressedCache.decode_step")
+        check(lib().da_decode_step(ref, device_stream(q.device)), "HybridCompressedCache.decode_step")
         if self.exact_seq_lens[layer_idx] >= self.exact_window_size:
             self.max_packed_len[layer_idx] += 1
             if self.total_seq_lens[layer_idx] % 256 == 0:  # reconcile with the device (:219-221)
                 self.max_packed_len[layer_idx] = int(self.packed_lengths[layer_idx].max().item())
         self.exact_seq_lens[layer_idx] += 1
         self.total_seq_lens[layer_idx] += 1
-        return out.unsqueeze(2)
+        return out
 
     def get_seq_length(self, layer_idx: int = 0) -> int:
         return self.total_seq_lens[layer_idx]

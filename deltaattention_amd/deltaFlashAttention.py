@@ -14,7 +14,7 @@ import ctypes
 import torch
 
 from ._launch import HALF, KernelLauncher, tensor, unit_stride
-from ._native import DA_F32, DA_I32, DA_VARIANT, check, dtype_code, lib, strides_array
+from ._native import DA_F32, DA_I32, DA_VARIANT, check, current_stream, dtype_code, lib, strides_array
 
 __all__ = ["hybrid_compressed_flash_kernel", "hybrid_compressed_flash_kernel_sanity",
            "pure_phase1_flash_kernel"]
@@ -75,7 +75,7 @@ class _HybridKernel(KernelLauncher):
             ts.data_ptr(), cnt.data_ptr(), DA_F32 if cnt.dtype == torch.float32 else DA_I32,
             out.data_ptr(), dtype_code(q, kd, vd, kp, vp, out), B, H, H, nq, nk, D, st, P, None, int(a["denseWindowSize"]),
             ctypes.c_float(float(a["sm_scale"])), DA_VARIANT[self.variant], 0, ws.data_ptr(),
-            ws_bytes, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            ws_bytes, ctypes.c_void_p(current_stream()))
         check(rc, self.NAME)
 
 

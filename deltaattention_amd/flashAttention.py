@@ -11,7 +11,7 @@ import torch
 
 from . import ops
 from ._launch import HALF, KernelLauncher, tensor, unit_stride
-from ._native import check, dtype_code, lib, strides_array
+from ._native import check, current_stream, dtype_code, lib, strides_array
 
 __all__ = ["triton_flash_attention", "_attn_fwd_flat"]
 
@@ -46,7 +46,7 @@ class _AttnFwdFlat(KernelLauncher):
         rc = lib().da_dense_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dtype_code(q, k, v, o),
                                     Z, H, H, N, N, D, st, 1 if a["IS_CAUSAL"] else 0,
                                     ctypes.c_float(float(a["sm_scale"])),
-                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+                                    ctypes.c_void_p(current_stream()))
         check(rc, "_attn_fwd_flat")
 
 

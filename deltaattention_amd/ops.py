@@ -17,7 +17,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _native
-from ._native import DA_F32, DA_I32, DA_VARIANT, check, dtype_code, lib, strides_array
+from ._native import DA_F32, DA_I32, DA_VARIANT, check, current_stream, dtype_code, lib, strides_array
 
 __all__ = ["PackedKV", "chunking", "select", "pack", "hybrid_prefill", "dense_prefill",
            "delta_prefill", "VarlenBatch", "varlen_batch", "PackedVarlen", "select_varlen",
@@ -25,7 +25,7 @@ __all__ = ["PackedKV", "chunking", "select", "pack", "hybrid_prefill", "dense_pr
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(current_stream())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

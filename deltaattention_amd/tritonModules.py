@@ -10,13 +10,13 @@ import ctypes
 import torch
 
 from ._launch import HALF, KernelLauncher, tensor, unit_stride
-from ._native import check, dtype_code, lib
+from ._native import check, current_stream, dtype_code, lib
 
 __all__ = ["chunked_eval_kernel", "parallel_scatter_pack_kv_kernel"]
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(current_stream())
 
 
 class _ChunkedEval(KernelLauncher):
