@@ -82,7 +82,6 @@ struct AttnArgs {
   const float* zeros;  // 64 zero biases (the exact tiles)
   int wcap;            // nblk_cap * 128
   int hpw;          // query heads per workgroup (4, 2 or 1)
-  int rows_per_wg;  // 256 / hpw
   int n_row_groups;
   int units;        // B * Hkv * (G / hpw)
   int slots;        // workgroups an XCD runs at once, two a CU
@@ -186,6 +185,10 @@ template <int N>
 __device__ __forceinline__ void lgkm_wait(u32x4& a, u32x4& b) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "i"(N));
 }
+template <int N>
+__device__ __forceinline__ void lgkm_wait(u32x4& a) {
+  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(a) : "i"(N));
+}
 // An unspecified value that costs no instruction: for a register array on a path where
 // it is dead, so that it is not live around the loop.
 template <typename T>
@@ -224,13 +227,18 @@ constexpr float kLazyLog2 = 8.0f;
 // 16 * 2^8: below that bound every p is at most 2^8 * 16, and a rescale is not needed
 // (p stays far from fp32's range and keeps bf16's relative precision).
 constexpr float kLazySum = 16.0f * 256.0f;
+// That (LAZY) is for GQA groups that are a multiple of 4.  The others take every tile's maximum:
+// the largest p of a row is then 1, which 16 bits hold exactly, and their error against 64
+// bits stays what it was (fp16, 8 heads x 1067 tokens: 2.58e-4; 4 % more with the lazy rule).
 
 // ====================================================================================
 // The 16-bit attention kernel, for every GQA group.
 //
 // A workgroup is 4 waves, one per SIMD: 4, 2 or 1 query heads of a GQA group (hpw) over 64,
-// 128 or 256 rows, each wave 64 rows of one head as two 32-row column blocks, so that every K
-// fragment and every V^T fragment read from LDS feeds two MFMAs.  Two workgroups share a CU:
+// 128 or 256 rows, each wave 64 rows of one head as two 32-row column blocks (NCB), so that
+// every K fragment and every V^T fragment read from LDS feeds two MFMAs.  Small grids take
+// half the rows, one column block a wave (launch_attn_rows; the rows' sums are the same bit for
+// bit), with the fragments read further ahead, since each feeds one MFMA.  Two workgroups share a CU:
 // while a wave runs its softmax (VALU), the other workgroup's wave on its SIMD has the matrix
 // pipe (its MFMAs go out at raised priority).  Tiles are 32 keys; every tile boundary falls
 // on the reference's logical 128-key grid.
@@ -250,8 +258,8 @@ constexpr float kLazySum = 16.0f * 256.0f;
 // 1.97 against 2.04 ms, 131072 27.9 / 28.7; ragged batches 4.5 / 4.7 ms).  It reads each tile
 // twice as often from L2, which costs up to 0.3 % where neither matters (dense 32768).  Groups
 // that are not a multiple of 4 ran a 32-row kernel that staged tiles through registers: 8000
-// tokens x 32 heads, keys repeated to the query heads, 233 against 318 us; dense 16384 x 32
-// heads of their own 1.85 against 2.70 ms.
+// tokens x 32 heads, keys repeated to the query heads, 286 against 319 us (236 with the lazy
+// maximum below).
 // ====================================================================================
 constexpr int kWTK = 32;                         // keys per tile
 constexpr int kWKBytes = kWTK * kD * 2;          // 8 KiB
@@ -313,10 +321,10 @@ __device__ __forceinline__ void item_at(int k, int units, int n_rg, int slots, i
 }
 
 // One (unit, row group) of attn_w64_kernel: a.hpw (4, 2 or 1) query heads of one (batch, KV
-// head) over 256 / hpw rows.  Ends with every LDS read of the window loop done (its last
+// head) over 128 NCB / hpw rows.  Ends with every LDS read of the window loop done (its last
 // barrier) and every load landed; the finalize uses only the wave's own Q region, so the next
 // item may start staging at once.
-template <int VARIANT, int DT>
+template <int VARIANT, int DT, int NCB, bool LAZY>
 __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit, const int rg) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* const kst0 = smem;
@@ -339,18 +347,18 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   const int g = gb / a.B, b = gb - (gb / a.B) * a.B;
   const int bg = b * a.Hkv + g;
   const int h = g * a.G + (hu << hsh) + (wid & ((1 << hsh) - 1));
-  const int wg_rows = 256 >> hsh;
+  const int wg_rows = (128 * NCB) >> hsh;
   const int R0 = rg * wg_rows;
   const int Nq = a.seq.cu ? a.seq.len(b) : a.Nq;
   const int Nk = a.seq.cu ? a.seq.len(b) : a.Nk;
   if (R0 >= Nq) return;  // a row group past the end of a shorter sequence (whole workgroup)
   // first row of this wave; column block cb holds r0w + 32 cb + ql
-  const int r0w = R0 + 64 * (wid >> hsh);
+  const int r0w = R0 + 32 * NCB * (wid >> hsh);
   const int wg_end = R0 + wg_rows;
 
   // ---- schedule: packed tiles 0 .. n1 - 1, then exact tiles from key ds on.  A workgroup's
   // rows lie in one logical 128-row block, except where one head takes 256 rows (hpw
-  // 1): its tiles are then the union of the two blocks' schedules, and a wave skips those
+  // 1, NCB 2): its tiles are then the union of the two blocks' schedules, and a wave skips those
   // that its own block (n1w, dsw) does not have ----
   int P = a.P_host;
   if (a.P_dev) P = min(a.seq.cu ? a.P_dev[b] : *a.P_dev, a.P_host);
@@ -373,7 +381,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     block_schedule(start_w, n1w, dsw);
     n1 = n1w;
     ds = dsw;
-    if (hsh == 0 && R0 + kBlock < Nq) {
+    if (NCB == 2 && hsh == 0 && R0 + kBlock < Nq) {
       int n2w, d2w;
       block_schedule(start_w ^ kBlock, n2w, d2w);
       n1 = max(n1, n2w);
@@ -385,7 +393,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     const int nblk = (P + kBlock - 1) / kBlock;
     const int32_t* from = a.sched + (int64_t)bg * 2 * a.nblk_cap + a.nblk_cap;
     int last;
-    safe_prefix(from, from, nblk, r0w + 64, n1w, last, lane);
+    safe_prefix(from, from, nblk, r0w + 32 * NCB, n1w, last, lane);
     safe_prefix(from, from, nblk, wg_end, n1, last, lane);
     n1w = min(n1w * (kBlock / kWTK), (P + kWTK - 1) / kWTK);
     n1 = min(n1 * (kBlock / kWTK), (P + kWTK - 1) / kWTK);
@@ -406,11 +414,10 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   constexpr bool kWeights = VARIANT == kHybrid || VARIANT == kPure;
 
   auto key0_of = [&](int t) { return t < n1 ? t * kWTK : ds + (t - n1) * kWTK; };
-  // causal: a Phase-2 tile whose first key is past the wave's last row (r0w + 63) is
-  // skipped; tiles n1 + (r0w + 63 - ds) / 32 + 1 onwards are
+  // causal: a Phase-2 tile whose first key is past the wave's last row is skipped
   int t_skip = INT_MAX;
   if (a.causal) {
-    const int d = r0w + 63 - ds;
+    const int d = r0w + 32 * NCB - 1 - ds;
     t_skip = __builtin_amdgcn_readfirstlane(d < 0 ? n1 : n1 + d / kWTK + 1);
   }
   if (kPureV) t_skip = __builtin_amdgcn_readfirstlane(n1w);
@@ -503,17 +510,19 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   int v_lane = (4 * ((lane >> 4) >> 1) + ((lane & 15) >> 2)) * 256 +
                ((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) << 4) + 8 * (lane & 1) + 64 * ((lane & 15) >> 2);
 
-  f32x16 o[2][4];
+  f32x16 o[NCB][4];
 #pragma unroll
-  for (int cb = 0; cb < 2; ++cb)
+  for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[cb][i] = f32x16{};
-  f32x16 s[2];
-  u32x4 pw[2][2];
+  f32x16 s[NCB];
+  u32x4 pw[NCB][2];
   // mc: the running maximum times c, the reference point of p = 2^(s c - mc).  Until a
   // lane has seen a finite score it is -FLT_MAX: every finite score then gives p = +inf
   // (the exact rule takes over), a masked one p = 0, and s c - mc is never NaN
-  float mc[2] = {-__FLT_MAX__, -__FLT_MAX__}, l_i[2] = {0.0f, 0.0f};
+  float mc[NCB], l_i[NCB];
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb) mc[cb] = -__FLT_MAX__, l_i[cb] = 0.0f;
   const float c = a.scale_log2;
 
   unsigned stA = 0, stB = kWKBytes;
@@ -527,9 +536,9 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   u32x4 qreg[kD / 16];
   {
     // both column blocks requested before either is used: one round trip, not two
-    u32x4 w[2][kD / 16];
+    u32x4 w[NCB][kD / 16];
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
+    for (int cb = 0; cb < NCB; ++cb) {
       const int row = r0w + 32 * cb + ql;
       const uint16_t* qrow = a.q + a.seq.base(b, a.sq_b, a.sq_n) + (int64_t)h * a.sq_h + (int64_t)min(row, Nq - 1) * a.sq_n;
 #pragma unroll
@@ -541,7 +550,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     // redefined so that the loop does not see Q as an outstanding load (the S = K Q^T
     // blocks would otherwise wait for every memory load, the staging loads included)
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
+    for (int cb = 0; cb < NCB; ++cb) {
       const int row = r0w + 32 * cb + ql;
 #pragma unroll
       for (int t = 0; t < kD / 16; ++t) {
@@ -559,8 +568,8 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     lds_barrier();
   }
 
-  constexpr int kWAhead = 3;    // V^T fragments read ahead of their MFMAs
-  constexpr int kWQKAhead = 2;  // (K, Q) fragment pairs read ahead of their MFMAs
+  constexpr int kWAhead = NCB == 2 ? 3 : 6;    // V^T fragments read ahead of their MFMAs
+  constexpr int kWQKAhead = NCB == 2 ? 2 : 5;  // (K, Q) fragment pairs (one block: K) read ahead
   const int nwin = T > 0 ? T + 1 : 0;
   // ---- matrix work of a window: O^T += V^T P^T for tile t - 1 (PV), then S^T = K Q^T for
   // tile t (QK), each LDS fragment feeding both column blocks ----
@@ -579,7 +588,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     constexpr int NM = NPV + NQK;                // MFMA pairs
     // stream element of MFMA pair i; elements issued before pair i's wait
     constexpr auto el = [](int i) { return i < NPV ? i : EQK + (i - NPV); };
-    constexpr auto size = [](int e) { return (BIAS && e == EBIAS) ? 4 : 2; };
+    constexpr auto size = [](int e) { return (BIAS && e == EBIAS) ? 4 : e >= EQK ? NCB : 2; };
     constexpr auto issued = [el](int i) {
       int n = 0;
       for (int k = 0; k <= i; ++k) {
@@ -606,11 +615,11 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     if constexpr (QK) {
       asm volatile("" : "+v"(k_lane));
       kla = lds_addr(kst0) + stA + k_lane;
-      qla = lds_addr(qs) + k_lane;
+      if constexpr (NCB == 2) qla = lds_addr(qs) + k_lane;
       bla = lds_addr(meta_of(t) + kWCnt) + 16 * hl;
     }
     i16x4 vlo[8], vhi[8];
-    u32x4 kw[kD / 16], qw[kD / 16], bw[4];
+    u32x4 kw[kD / 16], qw[NCB == 2 ? kD / 16 : 1], bw[4];
     auto read = [&](auto EC) {
       constexpr int e = decltype(EC)::value;
       if constexpr (e < NPV) {
@@ -622,7 +631,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
       } else {
         constexpr int j = e - EQK;
         kw[j] = ds_read_b128_asm(kla ^ (32u * j));
-        qw[j] = ds_read_b128_asm(qla ^ (32u * j));
+        if constexpr (NCB == 2) qw[j] = ds_read_b128_asm(qla ^ (32u * j));
       }
     };
     static_for<issued(0)>(read);
@@ -632,10 +641,11 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
         lgkm_wait<pending(i)>(vlo[i], vhi[i]);
         const u32x4 vw = __builtin_bit_cast(u32x4, __builtin_shufflevector(vlo[i], vhi[i], 0, 1, 2, 3, 4, 5, 6, 7));
         o[0][i & 3] = E16<DT>::mfma(vw, pw[0][i >> 2], o[0][i & 3]);
-        o[1][i & 3] = E16<DT>::mfma(vw, pw[1][i >> 2], o[1][i & 3]);
+        if constexpr (NCB == 2) o[1][i & 3] = E16<DT>::mfma(vw, pw[1][i >> 2], o[1][i & 3]);
       } else {
         constexpr int j = i - NPV;
-        lgkm_wait<pending(i)>(kw[j], qw[j]);
+        if constexpr (NCB == 2) lgkm_wait<pending(i)>(kw[j], qw[j]);
+        else lgkm_wait<pending(i)>(kw[j]);
         if constexpr (j == 0) {
           // S^T starts at the keys' biases (read before pair 0, so complete now),
           // or at zero (the MFMA's inline constant)
@@ -647,14 +657,14 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
                                                       __builtin_shufflevector(b2, b3, 0, 1, 2, 3, 4, 5, 6, 7),
                                                       0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
             s[0] = E16<DT>::mfma(kw[0], qreg[0], c0);
-            s[1] = E16<DT>::mfma(kw[0], qw[0], c0);
+            if constexpr (NCB == 2) s[1] = E16<DT>::mfma(kw[0], qw[0], c0);
           } else {
             s[0] = E16<DT>::mfma(kw[0], qreg[0], f32x16{});
-            s[1] = E16<DT>::mfma(kw[0], qw[0], f32x16{});
+            if constexpr (NCB == 2) s[1] = E16<DT>::mfma(kw[0], qw[0], f32x16{});
           }
         } else {
           s[0] = E16<DT>::mfma(kw[j], qreg[j], s[0]);
-          s[1] = E16<DT>::mfma(kw[j], qw[j], s[1]);
+          if constexpr (NCB == 2) s[1] = E16<DT>::mfma(kw[j], qw[j], s[1]);
         }
       }
       static_for<issued(i + 1 < NM ? i + 1 : i) - issued(i)>([&](auto K) {
@@ -667,7 +677,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
     const char* ms = meta_of(t);
     const int key0 = key0_of(t);
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
+    for (int cb = 0; cb < NCB; ++cb) {
       const int row = r0w + 32 * cb + ql;
       if (kPureV) {
         mask_pure32(s[cb], (const int*)(ms + kWTs), row, hl);
@@ -696,22 +706,24 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
       return psa + psb;
     };
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      float ps = exps(cb, -mc[cb]);
+    for (int cb = 0; cb < NCB; ++cb) {
+      float ps = LAZY ? exps(cb, -mc[cb]) : 0.0f;
       // the bound also catches an infinite sum
-      if (__builtin_amdgcn_ballot_w64(ps > kLazySum)) {
+      if (!LAZY || __builtin_amdgcn_ballot_w64(ps > kLazySum)) {
         float m = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; r += 2) m = __builtin_fmaxf(m, __builtin_fmaxf(s[cb][r], s[cb][r + 1]));
         const float mxc = halves_max(m) * c;
         // alpha = 1 exactly where a lane keeps its maximum (also where it has none yet)
-        const bool upd = mxc > mc[cb] + kLazyLog2;
+        const bool upd = mxc > mc[cb] + (LAZY ? kLazyLog2 : 0.0f);
         const float m_new = upd ? mxc : mc[cb];
         const float alpha = upd ? exp2_fast(mc[cb] - m_new) : 1.0f;
+        if (LAZY || __builtin_amdgcn_ballot_w64(upd)) {
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
+          for (int db = 0; db < 4; ++db)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[cb][db][r] *= alpha;
+            for (int r = 0; r < 16; ++r) o[cb][db][r] *= alpha;
+        }
         l_i[cb] *= alpha;
         mc[cb] = m_new;
         ps = exps(cb, -m_new);
@@ -777,7 +789,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   // whole rows, four per store instruction, instead of 16 bytes of 32 rows ----
   uint16_t* const obase = a.out + a.seq.base(b, a.so_b, a.so_n) + (int64_t)h * a.so_h;
 #pragma unroll
-  for (int cb = 0; cb < 2; ++cb) {
+  for (int cb = 0; cb < NCB; ++cb) {
     const float l_tot = halves_sum(l_i[cb]);
     float inv;
     if (VARIANT == kPure)
@@ -816,18 +828,18 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   }
 }
 
-// Work distribution.  Static (a.queue null, the dense control): workgroup i runs on XCD
+// Work distribution.  Static (a.queue null, the dense control and small grids): workgroup i runs on XCD
 // i mod 8 and takes one item; when the units split evenly over the 8 XCDs, each XCD gets
 // a contiguous range of units and walks their row groups longest first, so a unit's K/V
-// stay in one XCD's L2.  Persistent (a.queue set, the hybrid, sanity and pure Phase 1
-// variants, whose schedule kernel zeroes the 8 counters just before): two workgroups per
+// stay in one XCD's L2.  Persistent (a.queue set, large grids of the hybrid, sanity and
+// pure Phase 1 variants, whose schedule kernel zeroes the 8 counters just before): two workgroups per
 // CU loop over items.  Queue q holds the units of XCD q's static share in the same
 // order (unit by unit, longest row group first) and a.queue[q] counts the items taken;
 // a workgroup takes from the queue of the XCD it runs on and, once that is empty, from
 // the others, so the XCDs, whose clocks differ by several per cent, finish together,
 // and no dispatch gap lies between two items on a CU.  Every counter only grows, so each
 // workgroup's loop ends after at most 8 empty takes; workgroups never wait on each other.
-template <int VARIANT, int DT>
+template <int VARIANT, int DT, int NCB, bool LAZY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_w64_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -892,9 +904,9 @@ void attn_w64_kernel(AttnArgs a) {
         (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(ap));
     const AttnArgs ai = *ap;
-    attn_w64_item<VARIANT, DT>(ai, unit, rg);
+    attn_w64_item<VARIANT, DT, NCB, LAZY>(ai, unit, rg);
 #else
-    attn_w64_item<VARIANT, DT>(a, unit, rg);
+    attn_w64_item<VARIANT, DT, NCB, LAZY>(a, unit, rg);
 #endif
   }
 }
@@ -1337,22 +1349,50 @@ static int cu_count() {
   return n[dev];
 }
 
-template <int V, int DT>
-static int launch_attn_t(AttnArgs& a, hipStream_t st) {
+// Items (the units times their row groups) of attn_w64_kernel with ncb column blocks a wave.
+static int64_t attn_items(const AttnArgs& a, int ncb) {
+  const int rows = 128 * ncb / a.hpw;
+  return (int64_t)((a.Nq + rows - 1) / rows) * a.units;
+}
+
+template <int V, int DT, int NCB, bool LAZY>
+static int launch_attn_cb(AttnArgs& a, hipStream_t st) {
   static int done = 0;
   if (!done) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_w64_kernel<V, DT>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_w64_kernel<V, DT, NCB, LAZY>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kWLds);
     if (e != hipSuccess) return set_error(DA_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     done = 1;
   }
   a.slots = 2 * cu_count() / 8;
-  const int64_t items = (int64_t)a.n_row_groups * a.units;
+  const int64_t items = attn_items(a, NCB);
+  a.n_row_groups = (int)(items / a.units);
   // persistent: as many workgroups as run at once (two a CU) take items until the queues are
-  // empty; static: one workgroup per item
-  const unsigned grid = (unsigned)(a.queue ? std::min<int64_t>(items, 2 * cu_count()) : items);
-  hipLaunchKernelGGL((attn_w64_kernel<V, DT>), dim3(grid), dim3(256), kWLds, st, a);
+  // empty; static: one workgroup per item, also for the hybrid variants where all of them run at
+  // once (nothing is left to take, and each workgroup's looks at eight queues, one after the
+  // other, cost 4 to 16 us: delta step of 1531 tokens 82.5 -> 78.9, of 4090 127 -> 110) and with
+  // 32 rows a wave (items are short: 2300 tokens 111 -> 73)
+  if (items <= 2 * cu_count() || NCB == 1) a.queue = nullptr;
+  const unsigned grid = (unsigned)(a.queue ? 2 * cu_count() : items);
+  hipLaunchKernelGGL((attn_w64_kernel<V, DT, NCB, LAZY>), dim3(grid), dim3(256), kWLds, st, a);
   return check_launch("attention kernel");
+}
+
+template <int V, int DT, bool LAZY>
+static int launch_attn_rows(AttnArgs& a, hipStream_t st) {
+  // Up to two 64-row items a CU, 32 rows a wave: a CU then has its two or four workgroups' worth
+  // of waves where it had one or two, and the longest item takes half the matrix and softmax
+  // work.  Dense, 32 heads in groups of 4: 1024 tokens 29.4 against 44.0 us, 2048 53 / 80, 4096
+  // 139 / 163, beyond the line 6000 302 / 286, 8000 508 / 444; delta step of 1531 tokens 64.9 /
+  // 78.9, 2300 73 / 87, beyond 6000 168 / 171, 8190 248 / 242; heads of their own, 1067 tokens x
+  // 32 37 / 52.
+  return attn_items(a, 2) <= 2 * cu_count() ? launch_attn_cb<V, DT, 1, LAZY>(a, st)
+                                            : launch_attn_cb<V, DT, 2, LAZY>(a, st);
+}
+
+template <int V, int DT>
+static int launch_attn_t(AttnArgs& a, hipStream_t st) {
+  return a.hpw == 4 ? launch_attn_rows<V, DT, true>(a, st) : launch_attn_rows<V, DT, false>(a, st);
 }
 
 template <int DT>
@@ -1425,10 +1465,8 @@ static int fill_common(AttnArgs& a, const void* q, const void* k, const void* v,
   a.D = (int)D;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.hpw = (a.G % 4 == 0) ? 4 : (a.G % 2 == 0 ? 2 : 1);
-  a.rows_per_wg = 256 / a.hpw;
-  a.n_row_groups = (int)((Nq + a.rows_per_wg - 1) / a.rows_per_wg);
   a.units = (int)(B * Hkv * (a.G / a.hpw));
-  DA_REQUIRE((int64_t)a.n_row_groups * a.units < (1ll << 31), "%s: grid too large", who);
+  DA_REQUIRE(attn_items(a, 2) < (1ll << 31), "%s: grid too large", who);
   return DA_OK;
 }
 

@@ -71,3 +71,26 @@ def test_pure_phase1_unsorted_timestamps(gpu):
                              torch.from_numpy(cnt).to(gpu), window=64, variant="pure_phase1")
     _close(out, O.hybrid_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), kp.float().numpy(),
                                    vp.float().numpy(), ts, cnt, 64, variant="pure_phase1"))
+
+
+@pytest.mark.parametrize("variant", ["hybrid", "sanity", "pure_phase1", "dense"])
+@pytest.mark.parametrize("Hq,Hkv,N,D,W,dtype", [
+    (3, 3, 255, 64, 0, torch.bfloat16), (2, 2, 385, 128, 64, torch.float16), (5, 1, 900, 8, 128, torch.bfloat16),
+    (6, 3, 129, 128, 0, torch.bfloat16), (8, 1, 65, 128, 64, torch.float16), (12, 3, 193, 72, 64, torch.bfloat16),
+    (8, 2, 1400, 128, 128, torch.bfloat16)])
+def test_32_row_waves_match_64_row_ones(gpu, variant, Hq, Hkv, N, D, W, dtype):
+    """A grid of at most one workgroup a CU takes 32 rows a wave instead of 64.  Every row's sums
+    are the same: a batch of copies, which fills the chip, repeats the one sequence's output
+    bit for bit."""
+    from deltaattention_amd import ops, synth
+    q, k, v = synth.make_layer_inputs(1, Hq, Hkv, N, D, seed=N, dtype=dtype, device=str(gpu))
+    copies = 1 + 256 // Hkv  # more units than CUs, whatever the rows
+    qb, kb, vb = (x.repeat(copies, 1, 1, 1) for x in (q, k, v))
+    announce(f"32- and 64-row waves {variant} Hq={Hq} Hkv={Hkv} N={N} D={D} W={W} {dtype}")
+    if variant == "dense":
+        one, many = ops.dense_prefill(q, k, v), ops.dense_prefill(qb, kb, vb)
+    else:
+        tau = 9.0 * (D / 128) ** 0.5
+        one, many = (ops.delta_prefill(x, y, z, tau, 100, window=W, variant=variant)
+                     for x, y, z in ((q, k, v), (qb, kb, vb)))
+    assert torch.equal(one.expand_as(many), many)
