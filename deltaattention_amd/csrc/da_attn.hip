@@ -1156,7 +1156,9 @@ void attn_f32_kernel(AttnArgs a, int paired) {
     int n_safe, last;
     safe_prefix(bmax, bmax + a.nblk_cap, nblk, start_m - a.window, n_safe, last, lane);
     ds = max(0, ((last + 1) / kBlock) * kBlock);
-    if (VARIANT == kHybrid) n1 = min(n_safe * kBlock, a.wcap);
+    // not past P: a partly filled last block counts as safe where start_m - window > Nk + 1
+    // (more queries than keys), and a tile without a packed row has no row to load
+    if (VARIANT == kHybrid) n1 = min(n_safe * kBlock, P);
   } else if (VARIANT == kPure) {
     // the packed blocks up to the last that holds a key at or before the last row
     const int32_t* from = a.sched + (int64_t)bg * 2 * a.nblk_cap + a.nblk_cap;

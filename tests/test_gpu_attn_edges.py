@@ -94,3 +94,40 @@ def test_32_row_waves_match_64_row_ones(gpu, variant, Hq, Hkv, N, D, W, dtype):
         one, many = (ops.delta_prefill(x, y, z, tau, 100, window=W, variant=variant)
                      for x, y, z in ((q, k, v), (qb, kb, vb)))
     assert torch.equal(one.expand_as(many), many)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("variant", ["hybrid", "sanity", "pure_phase1"])
+@pytest.mark.parametrize("Hq,Hkv,Nq,Nk,P,W", [(4, 2, 1024, 256, 70, 64), (8, 2, 900, 130, 33, 0), (3, 3, 700, 100, 1, 64)])
+def test_more_queries_than_keys(gpu, variant, Hq, Hkv, Nq, Nk, P, W, dtype):
+    """Query blocks with start_m - W > Nk + 1 take the partly filled last packed block: its
+    rows past P weigh nothing and are not read (here they are NaN, in views of wider buffers).
+    The oracle has them as zero rows of count 0 and timestamp Nk + 1, which is what the
+    reference's masked loads give (deltaFlashAttention.py:70, 84-90)."""
+    from deltaattention_amd import ops, synth
+    D, room = 128, 256
+    q = synth.make_layer_inputs(1, Hq, Hkv, Nq, D, seed=Nq, dtype=dtype)[0]
+    _, k, v = synth.make_layer_inputs(1, Hq, Hkv, Nk, D, seed=Nk, dtype=dtype)
+    at = torch.linspace(0, Nk - 1, P).long()
+    ts = at.to(torch.int32).expand(1, Hkv, P)
+    cnt = torch.randint(1, 5, (1, Hkv, P), generator=torch.Generator().manual_seed(P), dtype=torch.int32)
+
+    def wide(x, fill):
+        buf = torch.full((*x.shape[:2], room, *x.shape[3:]), fill, dtype=x.dtype, device=gpu)
+        buf[:, :, :P] = x.to(gpu)
+        return buf[:, :, :P]
+    announce(f"more queries than keys {variant} Nq={Nq} Nk={Nk} P={P} W={W} {dtype}")
+    out = ops.hybrid_prefill(q.to(gpu), k.to(gpu), v.to(gpu), wide(k[:, :, at], float("nan")),
+                             wide(v[:, :, at], float("nan")), wide(ts, -1), wide(cnt, 1 << 20), window=W,
+                             variant=variant).float().cpu().numpy()
+    n = -(-P // 128) * 128 - P
+    pad = lambda x, fill: np.pad(x, [(0, 0), (0, 0), (0, n)] + [(0, 0)] * (x.ndim - 3), constant_values=fill)
+    kf, vf = k.float().numpy(), v.float().numpy()
+    want = O.hybrid_attention(q.float().numpy(), kf, vf, pad(kf[:, :, at.numpy()], 0), pad(vf[:, :, at.numpy()], 0),
+                              pad(ts.numpy(), Nk + 1), pad(cnt.numpy(), 0), W, variant=variant)
+    # a block past every key of both phases has no weight at all: 0 / 0 in the reference
+    some = np.isfinite(want)
+    assert np.isfinite(out)[some].all()
+    err = np.abs(out - want)[some]
+    bars = (2e-5, 2e-6) if dtype == torch.float32 else (2e-2, 1e-3)
+    assert err.max() <= bars[0] and err.mean() <= bars[1], (err.max(), err.mean())
