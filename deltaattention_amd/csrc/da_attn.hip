@@ -1109,29 +1109,37 @@ void attn_f32_kernel(AttnArgs a, int paired) {
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hl = lane >> 5, ql = lane & 31;
   // ---- workgroup -> (head, row block): whole heads per XCD where they split evenly, the
-  // longest row blocks first.  A grid of at most two workgroups a CU (paired) starts all at
-  // once, each CU taking one of the first half and one of the second: there the second half
-  // runs from the shortest up, so that every CU gets about the same work (2048 tokens x 8
-  // heads of 64 dims: 63 us, 80 with the longest first throughout) ----
+  // longest row blocks first.  Heads are numbered head-major, so that an XCD's share of a
+  // ragged batch is some heads of every sequence: with some sequences' heads instead, a long
+  // one among short ones had one XCD of eight (4096 + 15 x 64 tokens, 32 heads, dense: 12.7
+  // against 1.64 ms).  A grid of at most two workgroups a CU (paired) starts all at once, each
+  // CU taking one of the first half and one of the second: there the second half runs from the
+  // shortest up, so that every CU gets about the same work (2048 tokens x 8 heads of 64 dims:
+  // 63 us, 80 with the longest first throughout) ----
   const int nrb = (a.Nq + kFRows - 1) / kFRows;
   const int units = a.B * a.Hq;
-  int unit, rb;
+  const bool whole = (units & 7) == 0 && (!a.seq.cu || (a.Hq & 7) == 0);
+  int unit, j;  // j: row blocks from the last one
   if (paired) {
-    const int nx = (units & 7) == 0 ? 8 : 1;
+    const int nx = whole ? 8 : 1;
     const int upx = units / nx, n = upx * nrb;  // an XCD's heads and workgroups
     const int idx = blockIdx.x / nx, half = (n + 1) >> 1;
     const int e = idx < half ? idx : n - 1 - (idx - half);
     unit = (int)(blockIdx.x % nx) * upx + e % upx;
-    rb = nrb - 1 - e / upx;
-  } else if ((units & 7) == 0) {
+    j = e / upx;
+  } else if (whole) {
     const int idx = blockIdx.x >> 3;
     unit = (blockIdx.x & 7) * (units >> 3) + idx / nrb;
-    rb = nrb - 1 - idx % nrb;
+    j = idx % nrb;
   } else {
     unit = blockIdx.x % units;
-    rb = nrb - 1 - blockIdx.x / units;
+    j = blockIdx.x / units;
   }
-  const int h = unit % a.Hq, b = unit / a.Hq;
+  // without whole heads per XCD a long sequence's row blocks go round the XCDs (an odd number
+  // of units does that by itself)
+  if (a.seq.cu && !whole && !(units & 1)) unit = (unit + j) % units;
+  const int rb = nrb - 1 - j;
+  const int h = unit / a.B, b = unit % a.B;
   const int g = h / a.G;
   const int bg = b * a.Hkv + g;
   const int Nq = a.seq.cu ? a.seq.len(b) : a.Nq;

@@ -178,3 +178,36 @@ def test_varlen_variants_equal_per_sequence_runs(gpu, hq, hkv, variant):
         assert torch.equal(_per_seq(out, s, e), ref), f"{variant} sequence [{s}, {e})"
         ref = ops.dense_prefill(_per_seq(q, s, e), _per_seq(k, s, e), _per_seq(v, s, e))
         assert torch.equal(_per_seq(dense, s, e), ref), f"dense sequence [{s}, {e})"
+
+
+def _best_ms(fn):
+    fn()
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = float("inf")
+    for _ in range(5):
+        a.record()
+        fn()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (32, 8), (4, 4), (12, 4)])
+def test_fp32_long_sequence_uses_the_whole_chip(gpu, Hq, Hkv):
+    """One long sequence among short ones takes about as long as alone.  Its heads once lay on
+    one XCD of eight (8 heads: 3090 us, 400 alone)."""
+    from deltaattention_amd import ops, synth
+    lens = [4096] + [64] * 15
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    q, k, v = (x[0].transpose(0, 1).contiguous() for x in synth.make_layer_inputs(
+        1, Hq, Hkv, cu[-1], 128, seed=1, dtype=torch.float32, device=str(gpu)))
+    vb = ops.varlen_batch(cu, cu[-1], gpu)
+    one = [x[:lens[0]].transpose(0, 1)[None] for x in (q, k, v)]
+    announce(f"fp32 ragged {Hq}/{Hkv}")
+    alone = _best_ms(lambda: ops.dense_prefill(*one))
+    batch = _best_ms(lambda: ops.dense_prefill_varlen(q, k, v, vb))
+    print(f"alone {1e3 * alone:.0f} us, in the batch {1e3 * batch:.0f} us", flush=True)
+    assert batch <= 2.5 * alone
+    out = ops.dense_prefill_varlen(q, k, v, vb)
+    assert torch.equal(out[:lens[0]], ops.dense_prefill(*one)[0].transpose(0, 1))
