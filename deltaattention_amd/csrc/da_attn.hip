@@ -1365,6 +1365,14 @@ static int64_t attn_items(const AttnArgs& a, int ncb) {
   return (int64_t)((a.Nq + rows - 1) / rows) * a.units;
 }
 
+// Those of them that hold rows: a ragged batch's tokens as if its sequences were one.
+static int64_t attn_items_real(const AttnArgs& a, int ncb) {
+  const int64_t items = attn_items(a, ncb);
+  if (!a.seq.cu) return items;
+  const int rows = 128 * ncb / a.hpw;
+  return std::min<int64_t>(items, (int64_t)((a.seq.total + rows - 1) / rows) * (a.units / a.B));
+}
+
 template <int V, int DT, int NCB, bool LAZY>
 static int launch_attn_cb(AttnArgs& a, hipStream_t st) {
   static int done = 0;
@@ -1378,11 +1386,13 @@ static int launch_attn_cb(AttnArgs& a, hipStream_t st) {
   const int64_t items = attn_items(a, NCB);
   a.n_row_groups = (int)(items / a.units);
   // persistent: as many workgroups as run at once (two a CU) take items until the queues are
-  // empty; static: one workgroup per item, also for the hybrid variants where all of them run at
-  // once (nothing is left to take, and each workgroup's looks at eight queues, one after the
-  // other, cost 4 to 16 us: delta step of 1531 tokens 82.5 -> 78.9, of 4090 127 -> 110) and with
-  // 32 rows a wave (items are short: 2300 tokens 111 -> 73)
-  if (items <= 2 * cu_count() || NCB == 1) a.queue = nullptr;
+  // empty.  Only from more than four items a slot on, of which a quarter or more hold rows:
+  // before the queues gain anything each workgroup's looks at eight of them, and a take for every
+  // empty item of a ragged batch, cost more than they save (hybrid 8192 tokens, 1024 items: 276
+  // against 262 us static, sanity 107 / 81, 16384 tokens 171 / 160; 30 x 64 + 3500 + 200 tokens,
+  // 14080 items 958 of them with rows: 328 / 209)
+  const int64_t real = attn_items_real(a, NCB);
+  if (NCB == 1 || real <= 8 * cu_count() || 4 * real < items) a.queue = nullptr;
   const unsigned grid = (unsigned)(a.queue ? 2 * cu_count() : items);
   hipLaunchKernelGGL((attn_w64_kernel<V, DT, NCB, LAZY>), dim3(grid), dim3(256), kWLds, st, a);
   return check_launch("attention kernel");
@@ -1390,14 +1400,19 @@ static int launch_attn_cb(AttnArgs& a, hipStream_t st) {
 
 template <int V, int DT, bool LAZY>
 static int launch_attn_rows(AttnArgs& a, hipStream_t st) {
-  // Up to two 64-row items a CU, 32 rows a wave: a CU then has its two or four workgroups' worth
-  // of waves where it had one or two, and the longest item takes half the matrix and softmax
-  // work.  Dense, 32 heads in groups of 4: 1024 tokens 29.4 against 44.0 us, 2048 53 / 80, 4096
-  // 139 / 163, beyond the line 6000 302 / 286, 8000 508 / 444; delta step of 1531 tokens 64.9 /
-  // 78.9, 2300 73 / 87, beyond 6000 168 / 171, 8190 248 / 242; heads of their own, 1067 tokens x
-  // 32 37 / 52.
-  return attn_items(a, 2) <= 2 * cu_count() ? launch_attn_cb<V, DT, 1, LAZY>(a, st)
-                                            : launch_attn_cb<V, DT, 2, LAZY>(a, st);
+  // Up to two 64-row items a CU, 32 rows a wave.  Two workgroups a CU run at once either way, but
+  // the longest item, which the causal triangle's end waits for, takes half as long, and a chip
+  // that 64-row items fill by half is full.  Dense, 32 heads in groups of 4: 1024 tokens 29.4
+  // against 44.0 us, 2048 53 / 80, 4096 139 / 163, beyond the line 6000 302 / 286, 8000 508 / 444;
+  // delta step of 1531 tokens 64.9 / 78.9, 2300 73 / 87, beyond 6000 168 / 171, 8190 248 / 242;
+  // heads of their own, 1067 tokens x 32 37 / 52.  Without the causal mask all items are as long,
+  // and only the second reason is left: one item a CU (2048 tokens 72 / 83, 4096, two a CU, 260 /
+  // 228), unless half of a 64-row item would be past the rows (100 tokens x 16 x 32 heads of their
+  // own 17 / 20).  A ragged batch's items are counted by its tokens, not by the longest sequence (4096 +
+  // 15 x 64 tokens, dense, 12 heads in groups of 3: 149 / 246; 8 heads 109 / 172).
+  const bool short_gains = a.causal || attn_items(a, 1) == attn_items(a, 2);
+  return attn_items_real(a, 2) <= (short_gains ? 2 : 1) * cu_count() ? launch_attn_cb<V, DT, 1, LAZY>(a, st)
+                                                                    : launch_attn_cb<V, DT, 2, LAZY>(a, st);
 }
 
 template <int V, int DT>

@@ -193,21 +193,25 @@ def _best_ms(fn):
     return best
 
 
-@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (32, 8), (4, 4), (12, 4)])
-def test_fp32_long_sequence_uses_the_whole_chip(gpu, Hq, Hkv):
-    """One long sequence among short ones takes about as long as alone.  Its heads once lay on
-    one XCD of eight (8 heads: 3090 us, 400 alone)."""
+@pytest.mark.parametrize("dtype,Hq,Hkv,most", [
+    (torch.float32, 8, 8, 2.5), (torch.float32, 32, 8, 2.5), (torch.float32, 4, 4, 2.5), (torch.float32, 12, 4, 2.5),
+    (torch.bfloat16, 12, 4, 1.8), (torch.bfloat16, 3, 3, 1.8)])
+def test_long_sequence_uses_the_whole_chip(gpu, dtype, Hq, Hkv, most):
+    """One long sequence among short ones takes about as long as alone.  In fp32 its heads once
+    lay on one XCD of eight (8 heads: 3090 us, 400 alone); in 16 bits the empty items of the
+    short sequences were counted as work and it ran in items twice as long (12 heads: 246 us,
+    now 150, 110 alone)."""
     from deltaattention_amd import ops, synth
     lens = [4096] + [64] * 15
     cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
     q, k, v = (x[0].transpose(0, 1).contiguous() for x in synth.make_layer_inputs(
-        1, Hq, Hkv, cu[-1], 128, seed=1, dtype=torch.float32, device=str(gpu)))
+        1, Hq, Hkv, cu[-1], 128, seed=1, dtype=dtype, device=str(gpu)))
     vb = ops.varlen_batch(cu, cu[-1], gpu)
     one = [x[:lens[0]].transpose(0, 1)[None] for x in (q, k, v)]
-    announce(f"fp32 ragged {Hq}/{Hkv}")
+    announce(f"ragged {dtype} {Hq}/{Hkv}")
     alone = _best_ms(lambda: ops.dense_prefill(*one))
     batch = _best_ms(lambda: ops.dense_prefill_varlen(q, k, v, vb))
     print(f"alone {1e3 * alone:.0f} us, in the batch {1e3 * batch:.0f} us", flush=True)
-    assert batch <= 2.5 * alone
+    assert batch <= most * alone
     out = ops.dense_prefill_varlen(q, k, v, vb)
     assert torch.equal(out[:lens[0]], ops.dense_prefill(*one)[0].transpose(0, 1))
