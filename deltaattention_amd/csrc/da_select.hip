@@ -29,7 +29,9 @@
 // select_band_kernel instead, which decides most (anchor, row) pairs of a chunk from
 // matrix products, all at once, and leaves only the close ones to the exact tree.
 #include <algorithm>
+#include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "da_common.hpp"
 
@@ -37,7 +39,7 @@ namespace da {
 
 constexpr int kSelBatch = 32;
 constexpr int64_t kSelPairMinChunks = 2048;
-constexpr int64_t kBandMinRows = 96;
+constexpr int64_t kBandMinRows = 128;
 
 // x rounded to the 16-bit type DT (nearest even) and widened back to fp32.  For bf16
 // one v_cvt_pk_bf16_f32 with x in the high half and 0 in the low half leaves exactly
@@ -221,9 +223,21 @@ struct HalfKey<DA_F32> {
   static __device__ __forceinline__ float at(Row w, int i) { return w[i]; }
 };
 
-// select_step's decision for the row (x) and the anchor (a) a 32-lane half holds.
+// A half's row's norm as the cosine test takes it (tritonModules.py:48-54).
+template <int DT>
+__device__ __forceinline__ float half_norm(typename HalfKey<DT>::Row xb) {
+#pragma clang fp contract(off)
+  float p[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p[i] = HalfKey<DT>::at(xb, i) * HalfKey<DT>::at(xb, i);
+  return sqrt_rn(half_tree_sum<false, DT>(p[0], p[1], p[2], p[3]) + 1e-8f);
+}
+
+// select_step's decision for the row (x) and the anchor (a) a 32-lane half holds, with their
+// norms (the cosine test alone reads them).
 template <bool COS, bool A16, int DT>
-__device__ __forceinline__ bool half_keep(typename HalfKey<DT>::Row xb, typename HalfKey<DT>::Row ab, float thr) {
+__device__ __forceinline__ bool half_keep(typename HalfKey<DT>::Row xb, typename HalfKey<DT>::Row ab, float xn,
+                                          float an, float thr) {
 #pragma clang fp contract(off)
   float x[4], a[4], p[4];
 #pragma unroll
@@ -233,8 +247,6 @@ __device__ __forceinline__ bool half_keep(typename HalfKey<DT>::Row xb, typename
   }
   if constexpr (COS) {  // tritonModules.py:48-54
     const float dot = half_tree_sum<false, DT>(x[0] * a[0], x[1] * a[1], x[2] * a[2], x[3] * a[3]);
-    const float xn = sqrt_rn(half_tree_sum<false, DT>(x[0] * x[0], x[1] * x[1], x[2] * x[2], x[3] * x[3]) + 1e-8f);
-    const float an = sqrt_rn(half_tree_sum<false, DT>(a[0] * a[0], a[1] * a[1], a[2] * a[2], a[3] * a[3]) + 1e-8f);
     return __fdiv_rn(dot, xn * an) < thr;
   } else if constexpr (A16) {  // tritonModules.py:55-58 in the keys' 16-bit arithmetic
 #pragma unroll
@@ -251,6 +263,30 @@ __device__ __forceinline__ bool half_keep(typename HalfKey<DT>::Row xb, typename
     }
     return half_tree_sum<false, DT>(p[0], p[1], p[2], p[3]) > thr;
   }
+}
+template <bool COS, bool A16, int DT>
+__device__ __forceinline__ bool half_keep(typename HalfKey<DT>::Row xb, typename HalfKey<DT>::Row ab, float thr) {
+  return half_keep<COS, A16, DT>(xb, ab, COS ? half_norm<DT>(xb) : 0.0f, COS ? half_norm<DT>(ab) : 0.0f, thr);
+}
+
+// The lower halves of x and y side by side, then their upper ones.
+template <typename Row>
+__device__ __forceinline__ void swap_rows(const Row x, const Row y, Row& lower, Row& upper) {
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(Row) / 4); ++i) {
+    const auto xi = x[i], yi = y[i];  // scalars: a bit cast of the element itself takes element 0
+    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, xi),
+                                                     __builtin_bit_cast(uint32_t, yi), false, false);
+    const uint32_t lo = sw[0], up = sw[1];
+    using E = std::remove_cv_t<decltype(xi)>;
+    lower[i] = __builtin_bit_cast(E, lo);
+    upper[i] = __builtin_bit_cast(E, up);
+  }
+}
+__device__ __forceinline__ void swap_rows(const float x, const float y, float& lower, float& upper) {
+  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  lower = __uint_as_float(sw[0]);
+  upper = __uint_as_float(sw[1]);
 }
 
 // ---- two chunks per wave, one per 32-lane half ----
@@ -367,14 +403,18 @@ __global__ __launch_bounds__(256) void select_pair_kernel(
 //    next one, i.e. the 32 to 63 rows that follow each anchor.  With the rows' squared norms
 //    (fp32) each pair's distance (or cosine) follows to within a proven bound, and the pair
 //    is kept, dropped or open (three states, two bits, in the anchor's lane).
-// 2. The open pairs that come first in an anchor's row of bits are decided by the exact tree
-//    of the walk, two per wave and four such in one instruction stream, until every anchor's first kept
-//    row is known (about 0.4 pairs an anchor in bf16 arithmetic at one key in four kept,
-//    near none in fp32 arithmetic).
-// 3. Each wave follows the chain inside its 64 rows from all of them at once (pointer
-//    doubling between lanes), one wave joins the eight blocks.  An anchor that keeps none of
-//    the rows its tiles cover (or that 2 did not get to: keys all about as far apart as the
-//    threshold) scans on with the exact tree, eight rows a stream.
+// 2. Where these bits say that the rest would cost more than the serial walk (a wave's anchors
+//    have more open rows before their first kept one than kBandAhead, or more than kBandFar of
+//    them have no row at all: pairs about as far apart as the threshold, fp32 keys close together
+//    against their norms, one key in sixteen kept and fewer), all waves leave out 3.
+// 3. The open pairs that come first in an anchor's row of bits are decided by the exact tree
+//    of the walk, two per wave and four such in one instruction stream, until every anchor's first
+//    kept row is known (about 0.4 pairs an anchor in bf16 arithmetic at one key in four kept,
+//    near none in fp32 arithmetic); an anchor that keeps none of its tiles' rows looks at further
+//    tiles.  Both within a budget.
+// 4. Each wave follows the chain inside its 64 rows from all of them at once (pointer
+//    doubling between lanes), one wave joins the eight blocks.  Past an anchor whose next is not
+//    known (2, or 3's budget spent) that wave walks on, two rows a step, to the end of such blocks.
 //
 // Every decision is either proven by its bound or the exact tree's, so the result is the
 // walk's bit for bit.  The bounds, with u the unit roundoff of the walk's arithmetic:
@@ -390,14 +430,20 @@ __global__ __launch_bounds__(256) void select_pair_kernel(
 // * Rows with a norm at or above 2^120 (or infinite, or NaN) leave all their pairs open; a
 //   threshold below 1e-28 drops nothing, and nothing below 1e-30 is kept unseen.
 //
-// Measured, the selection alone, 8 heads of bf16 keys, one in four kept: 1531 keys 17 us
-// (71 with the serial walk), 32768 30 (75), 65536 50 (77, one in two); 8192 keys in one
-// chunk 0.22 ms (1.07).  What is left at few chunks is a chain of loads (the tiles, the
-// exact decisions' rows, five or six streams a wave); at many, reading the keys (75 of 108
-// us at 131072) and the exact decisions (32).
+// Measured, the selection alone, 8 heads, in brackets the serial walk.  bf16 keys in their own
+// arithmetic, one in four kept: 4096 keys 21 us (72), 32768 35 (73), 8192 in one chunk 0.24 ms
+// (1.07); one in eight 30 and 47, one in sixteen 64 and 83, one in 64 65 and 74, none 59 and 68:
+// from one in sixteen on most of it is the walk.  4096 fp32 keys: one in four 22 (60), none 54;
+// 32768 bf16 keys and the cosine test 24 (104), none 79.  What is left at few chunks is a chain of
+// loads (the tiles, the exact decisions' rows, five or six streams a wave).  Without 2 and the walk
+// in 4 one wave scanned on alone, eight rows a load: up to four times the serial walk's time.
 constexpr int kBandSeg = 512, kBandWaves = 8;
 constexpr int kBandEval = 4;     // exact decisions in one instruction stream, two each
-constexpr int kBandRounds = 24;  // streams a wave spends on its 64 anchors before it leaves the rest to 3
+constexpr int kBandRounds = 16;  // streams a wave spends on its 64 anchors
+constexpr int kBandAhead = 144;  // open rows before the first kept one, over a wave's anchors, that are too many
+constexpr int kBandFar = 6;      // anchors without a candidate in their tiles that are too many
+constexpr int kBandTiles = 4;    // more tiles it looks at for anchors whose own hold none
+constexpr int kWalkRows = 16;    // rows the walk loads ahead
 
 struct BandBounds {
   float c_lo, c_hi;  // e's lower and upper bound: c (n_a + n_c) - 2 g
@@ -510,9 +556,12 @@ void select_band_kernel(
     int32_t* __restrict__ chunk_counts, SeqMap seq, int64_t keep_sh, int divide_to) {
   __shared__ float s_norm[kBandWaves][2][32];     // a wave's candidates' norms (cosine: 1 / norm)
   __shared__ u32x2 s_path[kBandSeg];              // the chain from a row, inside its block of 64
-  __shared__ uint8_t s_to[kBandSeg];              // and where it leads
-  __shared__ uint8_t s_from[kBandSeg];
+  __shared__ int s_to[kBandSeg];                  // and where it leads, from the block's first row
+  __shared__ int s_from[kBandSeg];
   __shared__ uint64_t s_bits[kBandSeg / 64];
+  __shared__ u32x4 s_ku[kBandSeg];                // K and U of a row, put down while its wave looks at more tiles
+  __shared__ int s_hard[kBandWaves];              // the wave's tiles say that the walk is faster
+  __shared__ int s_left[kBandWaves];              // the wave left its anchors to the walk
   __shared__ int s_cur;
   const int D = FULL ? 128 : D_arg;
   const int tid = threadIdx.x;
@@ -553,72 +602,161 @@ void select_band_kernel(
   int cur = s;  // the next anchor
   int count = 0;
   const int seg = blockDim.x;  // rows a segment: 64 a wave
+  // the wave that joins the blocks and walks: another SIMD's for each of a CU's workgroups, in
+  // whatever order it gets them
+  const int lead = (int)((blockIdx.x >> 3) + (blockIdx.x >> 8)) % min(seg / 64, 4);
+  // ---- the walk of the rows from r on, two a step: both against the anchor, one a half, and
+  // the second against the first (of two steps at once), which does not wait for the anchor.
+  // Ends at the first anchor at or past `stop`, which it returns; the kept rows before go into
+  // s_bits (of the segment at sb). ----
+  auto walk_on = [&](Row a, int r, const int stop, const int sb) -> int {
+    float an = COS ? half_norm<DT>(a) : 0.0f;
+    Row x[kWalkRows / 2], y[kWalkRows / 2];
+    auto load = [&](Row (&v)[kWalkRows / 2], const int from) {
+      if (from + kWalkRows <= e) {
+        const Elem* p = base + (int64_t)(from + hl) * sk_n + (FULL ? 4 * ql : min(4 * ql, D - 4));
+#pragma unroll
+        for (int j = 0; j < kWalkRows / 2; ++j, p += 2 * sk_n) {
+          v[j] = *(const Row*)p;
+          if constexpr (!FULL) {
+#pragma unroll
+            for (int i = 0; i < (int)(sizeof(Row) / 4); ++i) v[j][i] = 4 * ql < D ? v[j][i] : 0;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < kWalkRows / 2; ++j) v[j] = row_bits(min(from + 2 * j + hl, e - 1));
+      }
+    };
+    load(x, r);
+    for (; r < e; r += kWalkRows) {
+      load(y, r + kWalkRows);
+      uint32_t bb = 0;
+#pragma unroll
+      for (int j = 0; j < kWalkRows / 2; j += 2) {
+        Row odd, even;  // rows 1 and 3, and 2 and 4, of these four
+        swap_rows(x[j], x[j + 1], odd, even);
+        float xn[2] = {}, on = 0.0f, en = 0.0f;
+        if constexpr (COS) {
+          xn[0] = half_norm<DT>(x[j]);
+          xn[1] = half_norm<DT>(x[j + 1]);
+          swap_rows(xn[0], xn[1], on, en);
+        }
+        const uint64_t kc = __ballot(half_keep<COS, A16, DT>(even, odd, en, on, thr));
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          Row first, second;
+          float n1 = 0.0f, n2 = 0.0f;
+          swap_rows(x[j + u], x[j + u], first, second);
+          if constexpr (COS) swap_rows(xn[u], xn[u], n1, n2);
+          const uint64_t ka = __ballot(half_keep<COS, A16, DT>(x[j + u], a, xn[u], an, thr));
+          const bool k12 = (kc >> (32 * u)) & 1ull;
+          const bool k1 = ka & 1ull, k2 = k1 ? k12 : (ka >> 32) & 1ull;
+          bb |= (uint32_t)k1 << (2 * (j + u)) | (uint32_t)k2 << (2 * (j + u) + 1);
+#pragma unroll
+          for (int i = 0; i < (int)(sizeof(Row) / 4); ++i) a[i] = k2 ? second[i] : k1 ? first[i] : a[i];
+          if constexpr (COS) an = k2 ? n2 : k1 ? n1 : an;
+        }
+      }
+      if (e - r < kWalkRows) bb &= (1u << (e - r)) - 1u;
+      const int in = stop - r;  // rows of this batch before `stop`
+      const uint32_t mine = in >= kWalkRows ? ~0u : in > 0 ? (1u << in) - 1u : 0u;
+      count += __builtin_popcount(bb & mine);
+      const int rel = r + lane - sb;
+      if (lane < kWalkRows && ((bb & mine) >> lane) & 1u)
+        atomicOr((unsigned long long*)&s_bits[rel >> 6], 1ull << (rel & 63));
+      if (bb & ~mine) return r + __builtin_ctz(bb & ~mine);
+#pragma unroll
+      for (int j = 0; j < kWalkRows / 2; ++j) x[j] = y[j];
+    }
+    return e;
+  };
   for (int sb = s; sb < e; sb += seg) {
     // opaque: what derives from the lane is formed here, not held in registers over the loop
-    asm volatile("" : "+v"(lane), "+v"(ql), "+v"(hl));
+    lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    ql = lane & 31;
+    hl = lane >> 5;
+    count = __builtin_amdgcn_readfirstlane(count);
     const int se = min(sb + seg, e);
     if (cur < se) {
       const int tb = sb + 64 * wid;  // the wave's anchors: tiles tb and tb + 32
-      if (tb < se && tb + 63 >= cur) {
-        BandTile<DT> x, y;
+      const bool active = tb < se && tb + 63 >= cur;
+      BandTile<DT> x, y;
+      // K, U: the kept and the open rows among those from tb + base to tb + end: the 64 from the
+      // anchor's tile on, or, where these hold none, the tile looked at last (base 64 and up)
+      uint64_t K = 0, U = 0;
+      int base = lane & 32;
+      auto window_end = [&]() { return base + (base < 64 ? 64 : 32); };
+      const bool mine = tb + lane >= cur && tb + lane < e;
+      constexpr uint32_t huge = 0x7b800000u;  // 2^120
+      auto is_bad = [](float n) { return (__float_as_uint(n) & 0x7fffffffu) >= huge; };
+      auto scaled = [](float n) { return COS ? __builtin_amdgcn_rsqf(n + 1e-8f) : n; };
+      // The kept and the open ones of a tile's rows (cand, its norms in s_norm[wid][j], its
+      // first row at tb + pos) against the lane's anchor, row ql of the tile in x
+      auto tile_bits = [&](const BandTile<DT>& cand, const int j, const float na, const bool bad,
+                           const uint32_t bad_rows, const int pos, uint32_t& kept, uint32_t& open) {
+        const f32x16 g = band_gram<DT>(cand, x);
+        uint32_t kb = 0, db = 0;
+        // S^T layout: the lane holds anchor ql and candidates 8 q + 4 hl + i
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 nc4 = *(const f32x4*)(&s_norm[wid][j][8 * q + 4 * hl]);
+          uint32_t kq = 0, dq = 0;  // the bits of these four: 1, 2, 4 and 8 need no register
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float dot = g[4 * q + i];
+            const uint32_t bit = 1u << i;
+            if (COS) {
+              const float sim = dot * (na * nc4[i]);
+              kq |= sim < bounds.keep ? bit : 0u;
+              dq |= sim > bounds.drop ? bit : 0u;
+            } else {
+              const float n2 = na + nc4[i];
+              kq |= __builtin_fmaf(n2, bounds.c_lo, -2.0f * dot) > bounds.keep ? bit : 0u;
+              dq |= __builtin_fmaf(n2, bounds.c_hi, -2.0f * dot) < bounds.drop ? bit : 0u;
+            }
+          }
+          asm("" : "+v"(kq), "+v"(dq));  // or the shift would go into the bits
+          kb |= kq << (8 * q);
+          db |= dq << (8 * q);
+        }
+        kb <<= 4 * hl;
+        db <<= 4 * hl;
+        kb |= __shfl_xor(kb, 32, 64);
+        db |= __shfl_xor(db, 32, 64);
+        const int lim = e - (tb + pos);  // rows of the tile before the chunk's end
+        const uint32_t valid = lim >= 32 ? ~0u : lim > 0 ? (1u << lim) - 1u : 0u;
+        const uint32_t sure = bad ? 0u : ~bad_rows;
+        kept = kb & valid & sure;
+        open = ~((kb | db) & sure) & valid;
+        __builtin_amdgcn_sched_barrier(0);  // one Gram tile's registers at a time
+      };
+      auto norms_written = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+      };
+      if (active) {
         load_tile(x, tb);
         load_tile(y, tb + 32);
         float nx = band_norm<DT>(x, ql, hl);
-        // K, U: the kept and the open rows among the 64 from the anchor's tile on
-        uint64_t K = 0, U = 0;
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
           // ---- anchors: the tile in x; candidates: x and y ----
           const float ny = band_norm<DT>(y, ql, hl);
           if (lane < 32) {
-            s_norm[wid][0][ql] = COS ? __builtin_amdgcn_rsqf(nx + 1e-8f) : nx;
-            s_norm[wid][1][ql] = COS ? __builtin_amdgcn_rsqf(ny + 1e-8f) : ny;
+            s_norm[wid][0][ql] = scaled(nx);
+            s_norm[wid][1][ql] = scaled(ny);
           }
-          const float na = COS ? __builtin_amdgcn_rsqf(nx + 1e-8f) : nx;
-          constexpr uint32_t huge = 0x7b800000u;  // 2^120
-          const bool bad = (__float_as_uint(nx) & 0x7fffffffu) >= huge;
-          const uint32_t bad0 = (uint32_t)__ballot(bad);
-          const uint32_t bad1 = (uint32_t)__ballot((__float_as_uint(ny) & 0x7fffffffu) >= huge);
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-          // S^T layout: the lane holds anchor ql and candidates 8 q + 4 hl + i of each tile
+          const uint32_t bad0 = (uint32_t)__ballot(is_bad(nx)), bad1 = (uint32_t)__ballot(is_bad(ny));
+          norms_written();
           uint32_t kept[2], open[2];
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const f32x16 g = band_gram<DT>(j == 0 ? x : y, x);
-            uint32_t kb = 0, db = 0;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const f32x4 nc4 = *(const f32x4*)(&s_norm[wid][j][8 * q + 4 * hl]);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const float dot = g[4 * q + i];
-                const uint32_t bit = 1u << (8 * q + i);
-                if (COS) {
-                  const float sim = dot * (na * nc4[i]);
-                  kb |= sim < bounds.keep ? bit : 0u;
-                  db |= sim > bounds.drop ? bit : 0u;
-                } else {
-                  const float n2 = na + nc4[i];
-                  kb |= __builtin_fmaf(n2, bounds.c_lo, -2.0f * dot) > bounds.keep ? bit : 0u;
-                  db |= __builtin_fmaf(n2, bounds.c_hi, -2.0f * dot) < bounds.drop ? bit : 0u;
-                }
-              }
-            }
-            kb <<= 4 * hl;
-            db <<= 4 * hl;
-            kb |= __shfl_xor(kb, 32, 64);
-            db |= __shfl_xor(db, 32, 64);
-            // candidates of this tile: after the anchor, before the chunk's end
-            const int lim = e - (tb + 32 * half + 32 * j);
-            uint32_t valid = lim >= 32 ? ~0u : lim > 0 ? (1u << lim) - 1u : 0u;
-            if (j == 0) valid &= ~((2u << ql) - 1u);
-            const uint32_t sure = bad ? 0u : ~(j == 0 ? bad0 : bad1);
-            kept[j] = kb & valid & sure;
-            open[j] = ~((kb | db) & sure) & valid;
-            __builtin_amdgcn_sched_barrier(0);  // one Gram tile's registers at a time
-          }
+          tile_bits(x, 0, scaled(nx), is_bad(nx), bad0, 32 * half, kept[0], open[0]);
+          tile_bits(y, 1, scaled(nx), is_bad(nx), bad1, 32 * half + 32, kept[1], open[1]);
+          const uint32_t after = ~((2u << ql) - 1u);  // candidates of the own tile: after the anchor
+          kept[0] &= after;
+          open[0] &= after;
           __builtin_amdgcn_wave_barrier();  // the norms are read before the next tile's are written
           if (half == 0) {
             x = y;
@@ -630,90 +768,143 @@ void select_band_kernel(
             U = open[0] | (uint64_t)open[1] << 32;
           }
         }
-        // ---- exact decisions, until every anchor's first candidate is a kept one ----
-        const bool mine = tb + lane >= cur && tb + lane < e;
-        for (int round = 0; round < kBandRounds; ++round) {
-          const uint64_t any = K | U;
-          const int first = any ? __builtin_ctzll(any) : 0;
-          uint64_t m = __ballot(mine && any != 0 && ((U >> first) & 1ull));
-          if (m == 0) break;
-          int l[2 * kBandEval];
-          Row ra[kBandEval], rx[kBandEval];
-          uint64_t kp[kBandEval];
-#pragma unroll
-          for (int i = 0; i < 2 * kBandEval; ++i) {
-            l[i] = m ? __builtin_ctzll(m) : l[i > 0 ? i - 1 : 0];
-            m &= m - 1ull;
-          }
-#pragma unroll
-          for (int i = 0; i < kBandEval; ++i) {
-            const int f0 = (l[2 * i] & 32) + __builtin_amdgcn_readlane(first, l[2 * i]);
-            const int f1 = (l[2 * i + 1] & 32) + __builtin_amdgcn_readlane(first, l[2 * i + 1]);
-            ra[i] = row_bits(tb + (hl ? l[2 * i + 1] : l[2 * i]));
-            rx[i] = row_bits(tb + (hl ? f1 : f0));
-          }
-#pragma unroll
-          for (int i = 0; i < kBandEval; ++i) kp[i] = __ballot(half_keep<COS, A16, DT>(rx[i], ra[i], thr));
-#pragma unroll
-          for (int i = 0; i < 2 * kBandEval; ++i)
-            if (lane == l[i]) {
-              U &= ~(1ull << first);
-              if ((kp[i >> 1] >> (32 * (i & 1))) & 1ull) K |= 1ull << first;
+        // Where the bounds decide little (pairs all about as far apart as the threshold, or close
+        // together against their norms) or the tiles hold too little (an anchor's next lies
+        // further on) the walk is faster, and the wave leaves its rows to it at once.
+        const float ahead = (float)__builtin_popcountll(U & ((K & (0ull - K)) - 1ull));
+        const bool far = __builtin_popcountll(__ballot(mine && (K | U) == 0 && tb + window_end() < e)) > kBandFar;
+        const bool open = __builtin_amdgcn_readfirstlane((int)wave_tree_sum_all(mine ? ahead : 0.0f)) > kBandAhead;
+        if (lane == 0) s_hard[wid] = far || open;
+      } else if (lane == 0) {
+        s_hard[wid] = 0;
+      }
+      __syncthreads();
+      if (active) {
+        // one such wave stands for all: none then holds the segment up with rows that the walk
+        // passes anyway (bf16 arithmetic, one key in eight kept: at most 128 open and none without
+        // a row in any wave; one in sixteen: above the line in every chunk)
+        bool hard = __ballot(lane < seg / 64 && s_hard[lane & (kBandWaves - 1)]) != 0;
+        int rounds = 0, tiles = 0;
+        while (!hard) {
+          // ---- exact decisions, until every anchor's first candidate is a kept one ----
+          for (;; ++rounds) {
+            const uint64_t any = K | U;
+            const int first = any ? __builtin_ctzll(any) : 0;
+            uint64_t m = __ballot(mine && any != 0 && ((U >> first) & 1ull));
+            if (m == 0) break;
+            if (rounds == kBandRounds) {
+              hard = true;
+              break;
             }
+            int l[2 * kBandEval];
+            Row ra[kBandEval], rx[kBandEval];
+            uint64_t kp[kBandEval];
+#pragma unroll
+            for (int i = 0; i < 2 * kBandEval; ++i) {
+              l[i] = m ? __builtin_ctzll(m) : l[i > 0 ? i - 1 : 0];
+              m &= m - 1ull;
+            }
+#pragma unroll
+            for (int i = 0; i < kBandEval; ++i) {
+              const int f0 = __builtin_amdgcn_readlane(base + first, l[2 * i]);
+              const int f1 = __builtin_amdgcn_readlane(base + first, l[2 * i + 1]);
+              ra[i] = row_bits(tb + (hl ? l[2 * i + 1] : l[2 * i]));
+              rx[i] = row_bits(tb + (hl ? f1 : f0));
+            }
+#pragma unroll
+            for (int i = 0; i < kBandEval; ++i) kp[i] = __ballot(half_keep<COS, A16, DT>(rx[i], ra[i], thr));
+#pragma unroll
+            for (int i = 0; i < 2 * kBandEval; ++i)
+              if (lane == l[i]) {
+                U &= ~(1ull << first);
+                if ((kp[i >> 1] >> (32 * (i & 1))) & 1ull) K |= 1ull << first;
+              }
+          }
+          // ---- the anchors whose rows so far hold none: tile after tile, until all have one ----
+          uint64_t want = __ballot(mine && (K | U) == 0 && tb + window_end() < e);
+          if (hard || want == 0) break;
+          s_ku[64 * wid + lane] = u32x4{(uint32_t)K, (uint32_t)(K >> 32), (uint32_t)U, (uint32_t)(U >> 32)};
+#pragma unroll 1
+          for (int half = 0; half < 2; ++half) {
+            if ((uint32_t)(want >> (32 * half)) == 0) continue;
+            load_tile(x, tb + 32 * half);
+            int pos = hl == half && ((want >> lane) & 1ull) ? window_end() : INT_MAX;  // the least of them
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) pos = min(pos, __shfl_xor(pos, d, 64));
+            pos = __builtin_amdgcn_readfirstlane(pos);
+            const float nx = band_norm<DT>(x, ql, hl);
+#pragma unroll 1
+            for (; tb + pos < e && tiles < kBandTiles; pos += 32, ++tiles) {
+              load_tile(y, tb + pos);
+              const float ny = band_norm<DT>(y, ql, hl);
+              if (lane < 32) s_norm[wid][1][ql] = scaled(ny);
+              const uint32_t bad1 = (uint32_t)__ballot(is_bad(ny));
+              norms_written();
+              uint32_t kept, open;
+              tile_bits(y, 1, scaled(nx), is_bad(nx), bad1, pos, kept, open);
+              __builtin_amdgcn_wave_barrier();
+              if (hl == half && ((want >> lane) & 1ull) && pos >= window_end()) {
+                base = pos;
+                s_ku[64 * wid + lane] = u32x4{kept, 0u, open, 0u};
+              }
+              want &= ~__ballot(hl == half && base == pos && (kept | open) != 0u);
+              if ((uint32_t)(want >> (32 * half)) == 0) break;
+            }
+          }
+          hard = tiles >= kBandTiles;
+          norms_written();
+          const u32x4 ku = s_ku[64 * wid + lane];
+          K = ku[0] | (uint64_t)ku[1] << 32;
+          U = ku[2] | (uint64_t)ku[3] << 32;
         }
         // ---- the chain inside the wave's 64 rows, from every row at once: path holds the
-        // anchors met from row l on, to is where it leaves them (64 ..), or 128 + the anchor
+        // anchors met from row l on, to is where it leaves them (64 and up), or -1 - the anchor
         // it stops at: one whose next is not known, to be looked for from row s_from on.
         // Six doublings cover 64 steps. ----
         const uint64_t any = K | U;
-        const int first = any ? __builtin_ctzll(any) : 64;
-        s_from[64 * wid + lane] = (uint8_t)((lane & 32) + first);
-        int to = any && !((U >> (first & 63)) & 1ull) ? (lane & 32) + first : 128 + lane;
+        const int first = any ? __builtin_ctzll(any) : 0;
+        const int at = any ? base + first : min(window_end(), e - tb);
+        s_from[64 * wid + lane] = at;
+        // (no next: past the block, where the chunk may end inside it)
+        int to = (any ? (U >> first) & 1ull : tb + at < e) ? -1 - lane : any ? at : max(at, 64);
         uint32_t lo = lane < 32 ? 1u << ql : 0u, hi = lane < 32 ? 0u : 1u << ql;
 #pragma unroll
         for (int d = 0; d < 6; ++d) {
-          const int src = to < 64 ? to : lane;
+          const int src = (unsigned)to < 64u ? to : lane;
           lo |= (uint32_t)__shfl((int)lo, src, 64);
           hi |= (uint32_t)__shfl((int)hi, src, 64);
           to = __shfl(to, src, 64);
         }
         s_path[64 * wid + lane] = u32x2{lo, hi};
-        s_to[64 * wid + lane] = (uint8_t)to;
+        s_to[64 * wid + lane] = to;
+        if (lane == 0) s_left[wid] = hard;
       }
       __syncthreads();
-      if (wid == 0) {
+      if (wid == lead) {
         // ---- the segment's chain: one lookup a block of 64 rows ----
         int p = cur - sb;
+        if (lane < seg / 64) s_bits[lane] = 0;
         for (int i = 0; i < seg / 64; ++i) {
           uint64_t bits = 0;
           while (p < 64 * (i + 1) && sb + p < se) {
             const u32x2 path = s_path[p];
-            const int to = __builtin_amdgcn_readfirstlane((int)s_to[p]);
+            const int to = __builtin_amdgcn_readfirstlane(s_to[p]);
             const uint64_t on = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(path[0]) |
                                 (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(path[1]) << 32;
             bits |= on;
             count += __builtin_popcountll(on);
-            if (to >= 128) {
-              // on from the anchor it stops at with the exact tree
-              const int pa = 64 * i + (to - 128);
-              const Row ra = row_bits(sb + pa);
-              int r = sb + 64 * i + __builtin_amdgcn_readfirstlane((int)s_from[pa]), at = e;
-              for (; r < e && at == e; r += 2 * kBandEval) {
-                Row rx[kBandEval];
-#pragma unroll
-                for (int u = 0; u < kBandEval; ++u) rx[u] = row_bits(min(r + 2 * u + hl, e - 1));
-#pragma unroll
-                for (int u = kBandEval - 1; u >= 0; --u) {  // the first of these rows that is kept
-                  const uint64_t kp = __ballot(half_keep<COS, A16, DT>(rx[u], ra, thr) && r + 2 * u + hl < e);
-                  if (kp) at = r + 2 * u + ((kp & 1ull) ? 0 : 1);
-                }
-              }
-              p = at - sb;
+            if (to < 0) {
+              // on from the anchor it stops at, past the blocks that were left to the walk
+              const int pa = 64 * i + (-1 - to);
+              int j = i + 1;
+              while (j < seg / 64 && __builtin_amdgcn_readfirstlane(s_left[j])) ++j;
+              p = walk_on(row_bits(sb + pa), sb + __builtin_amdgcn_readfirstlane(s_from[pa]) + 64 * i,
+                          min(sb + 64 * j, e), sb) - sb;
             } else {
               p = 64 * i + to;
             }
           }
-          if (lane == 0) s_bits[i] = bits;
+          if (lane == 0) s_bits[i] |= bits;
         }
         if (lane == 0) s_cur = sb + p;
       }
@@ -723,10 +914,10 @@ void select_band_kernel(
       if (tid < seg / 64) s_bits[tid] = 0;
       __syncthreads();
     }
-    if (sb + tid < se) keep_row[sb + tid] = (int32_t)((s_bits[tid >> 6] >> lane) & 1ull);
+    if (sb + 64 * wid + lane < se) keep_row[sb + 64 * wid + lane] = (int32_t)((s_bits[wid] >> lane) & 1ull);
     __syncthreads();  // the bits are read before the next segment's are written
   }
-  if (tid == 0) chunk_counts[w] = count;  // tritonModules.py:68-69
+  if (wid == lead && (threadIdx.x & 63) == 0) chunk_counts[w] = count;  // tritonModules.py:68-69
 }
 
 static int launch_select(const void* k, int dtype, int64_t B, int64_t Hkv, int64_t N, int64_t D, int64_t sk_b,
@@ -738,17 +929,17 @@ static int launch_select(const void* k, int dtype, int64_t B, int64_t Hkv, int64
   const int64_t total = B * Hkv * num_chunks;
   const int64_t blocks = (total + 3) / 4;
   DA_REQUIRE(blocks < (1ll << 31), "%s: too many chunks", who);
-  // The banded walk takes rows it can read 16 bytes at a time.  It spends a workgroup of a
-  // wave per 64 rows on a chunk, two or more at once on a CU, so its time grows with the
-  // chunks where the serial walks stay at 0.14 us a row until the SIMDs are full: the line
-  // lies where the times meet, at two rounds of the chip (bf16, 8 heads: 64 chunks of 512
-  // rows a head 23 against 71 us, 128 a head 50 against 77, 192 a head 79 against 76 at one
-  // key in eight kept; fp32 keys, which take a CU each: 64 a head 37 against 62, 128 a head
-  // 79 against 70; cosine: 240 a head 96 against 140).  Below 96 rows a chunk is too short
-  // to gain (64 rows: 24 against 20 us).
+  // The banded walk takes rows it can read 16 bytes at a time.  The line is one round of the chip:
+  // two workgroups a CU, one for fp32 keys (their registers).  There its time is 0.2 to 0.65 of
+  // the serial walk's with one key in two to eight kept and about the serial walk's with keys that
+  // it leaves to its own (0.8 to 1.05, the worst found 1.15: 512 chunks of bf16 keys, one in
+  // sixteen kept, 83 against 73 us).  A second round doubles the latter and gains little on the
+  // former: 1024 chunks 46 us at one key in two, 78 at one in eight, 103 and more from one in sixteen
+  // on, against 74; a look at a chunk's first 64 rows before the rest costs 6 us and leaves 97 to
+  // 165.  Below 128 rows a chunk is too short to gain (97 rows, 680 chunks: 19.5 against 17.1 us).
   const int per16 = dtype == DA_F32 ? 4 : 8;
   const int64_t rows = seq.cu && divide_to > 0 ? (N + divide_to - 1) / divide_to : std::min(chunk_size, N);
-  const int64_t band_max = (dtype == DA_F32 ? 512 : use_cosine ? 2048 : 1024) * std::max<int64_t>(1, kBandSeg / rows);
+  const int64_t band_max = dtype == DA_F32 ? 256 : 512;
   if (rows >= kBandMinRows && total <= band_max && (D & 7) == 0 && ((sk_b | sk_h | sk_n) % per16) == 0 &&
       ((uintptr_t)k & 15) == 0 && std::isfinite(threshold)) {
     const BandBounds bounds = band_bounds(use_cosine, a16, dtype, threshold);

@@ -537,6 +537,15 @@ def _band_keys(kind, H, N, D, dtype):
         k[0, :, torch.arange(N), torch.arange(N) % D] = 4.0
     elif kind == "constant":      # no key past a chunk's first is kept
         k = torch.randn((1, H, 1, D), generator=gen).expand(1, H, N, D)
+    elif kind == "plateaus":      # some anchors' next lies past the tiles compared, most do not
+        k = torch.randn((1, H, N, D), generator=gen)
+        for a in range(28, N - 40, 160):
+            k[:, :, a:a + 38] = k[:, :, a:a + 1]
+    elif kind == "mixed":         # stretches for the tiles between ones for the walk
+        k = torch.randn((1, H, N, D), generator=gen)
+        k[:, :, 700:1300] = k[:, :, 700:701]
+        k[:, :, 1500:1530] = k[:, :, 1500:1501]
+        k[:, :, 1900:] = k[:, :, 1900:].mul(0.02).cumsum(2)
     elif kind == "slow":          # few keys kept, far apart
         k = torch.randn((1, H, N, D), generator=gen).mul(0.05).cumsum(2)
     elif kind == "huge":          # norms past fp32's range beside ordinary rows
@@ -553,14 +562,18 @@ def _band_keys(kind, H, N, D, dtype):
     ("huge", 2, 700, 128, 300, "euclidean", 15.0), ("random", 3, 545, 96, 97, "euclidean", 13.5),
     ("random", 2, 545, 8, 545, "euclidean", 4.0), ("random", 2, 577, 128, 128, "euclidean", 1e-20),
     ("random", 2, 1300, 40, 0, "cosine", 0.1), ("slow", 2, 2100, 64, 700, "cosine", 0.99),
-    ("huge", 2, 700, 128, 300, "cosine", 0.1)])
+    ("huge", 2, 700, 128, 300, "cosine", 0.1), ("plateaus", 2, 1500, 128, 512, "euclidean", 13.0),
+    ("plateaus", 2, 1300, 128, 0, "cosine", 0.2), ("mixed", 2, 2600, 128, 2600, "euclidean", 13.0),
+    ("mixed", 2, 2600, 64, 1100, "euclidean", 9.0), ("mixed", 2, 2600, 128, 2600, "cosine", 0.3),
+    ("mixed", 3, 2600, 128, 130, "euclidean", 13.0)])
 @pytest.mark.parametrize("dtype,arith", [(torch.bfloat16, "native"), (torch.bfloat16, "fp32"),
                                          (torch.float16, "native"), (torch.float32, "native")],
                          ids=["bf16", "bf16-fp32", "fp16", "fp32"])
 def test_select_banded_walk(gpu, kind, H, N, D, chunk, metric, tau, dtype, arith):
     """The banded walk against the C oracle, bit for bit, where its shortcuts end: pairs all
     close to the threshold, anchors whose next lies past the tiles compared, rows its bounds
-    do not hold for, chunk lengths around its tiles and segments, every key type."""
+    do not hold for, blocks it leaves to the walk and takes up again, chunk lengths around its
+    tiles and segments, every key type."""
     from deltaattention_amd import ops
     k = _band_keys(kind, H, N, D, dtype)
     announce(f"banded select {kind} H={H} N={N} D={D} chunk={chunk} {metric} tau={tau} {dtype} {arith}")
@@ -570,3 +583,84 @@ def test_select_banded_walk(gpu, kind, H, N, D, chunk, metric, tau, dtype, arith
     got = keep.cpu().numpy()
     assert np.array_equal(got, ok), np.argwhere(got != ok)[:5]
     assert np.array_equal(cc.cpu().numpy(), occ)
+
+
+@pytest.mark.parametrize("metric,tau,arith", [("euclidean", 9.0, "native"), ("euclidean", 9.0, "fp32"),
+                                              ("cosine", 0.6, "native")])
+@pytest.mark.parametrize("dtype,H,N,chunk", [
+    (torch.float16, 3, 2000, 64), (torch.float16, 40, 8000, 512), (torch.bfloat16, 3, 2000, 64),
+    (torch.bfloat16, 40, 8000, 512), (torch.bfloat16, 80, 16000, 512), (torch.float16, 80, 16000, 512),
+    (torch.float32, 3, 2000, 64), (torch.float32, 40, 8000, 512)])
+def test_select_serial_walks(gpu, dtype, H, N, chunk, metric, tau, arith):
+    """The serial walks against the C oracle where the banded walk does not go: chunks of fewer
+    than 128 rows, more chunks than run at once (one chunk a wave, 640 of them) and 2560 (two a
+    wave, the 16-bit types)."""
+    from deltaattention_amd import ops, synth
+    k = synth.make_layer_inputs(1, H, H, N, 128, seed=31, rope_base=500000.0)[1].to(dtype)
+    announce(f"serial walk {dtype} H={H} N={N} chunk={chunk} {metric} {arith}")
+    keep, cc = ops.select(k.to(gpu), tau, chunk, 0, metric, arith=arith)
+    orac = "fp32" if arith == "fp32" else oracle_arith(k)
+    ok, occ = OC.select_delta(k.float().numpy(), tau, chunk, 0, metric, arith=orac)
+    assert np.array_equal(cc.cpu().numpy(), occ), "chunk counts differ"
+    assert np.array_equal(keep.cpu().numpy(), ok)
+
+
+@pytest.mark.parametrize("scale,tau", [(2e-3, 0.015), (40.0, 250.0)], ids=["subnormal-squares", "near-fp16-max"])
+def test_select_fp16_native_extremes_serial(gpu, scale, tau):
+    """The extremes of test_select_fp16_native_extremes on the walk of one chunk a wave (its four
+    heads take the banded walk): 640 chunks."""
+    from deltaattention_amd import ops, synth
+    k = (synth.make_layer_inputs(1, 40, 40, 8192, 128, seed=29, rope_base=10000.0)[1].float() * scale).to(torch.float16)
+    announce(f"select fp16 extremes, serial walk, scale={scale} tau={tau}")
+    keep, cc = ops.select(k.to(gpu), tau, 512, 0, arith="native")
+    ok, occ = OC.select_delta(k.float().numpy(), tau, 512, 0, arith="fp16")
+    assert np.array_equal(cc.cpu().numpy(), occ), "chunk counts differ"
+    assert np.array_equal(keep.cpu().numpy(), ok)
+
+
+@pytest.mark.parametrize("dtype,N,kind,tau,metric", [
+    (torch.bfloat16, 4096, "ar", 15.9, "euclidean"), (torch.bfloat16, 32768, "ar", 15.9, "euclidean"),
+    (torch.bfloat16, 65536, "ar", 15.9, "euclidean"), (torch.bfloat16, 32768, "constant", 0.5, "euclidean"),
+    (torch.bfloat16, 32768, "ar", -2.0, "cosine"), (torch.float16, 32768, "ar", 1e6, "euclidean"),
+    (torch.float32, 16384, "offset", 16.0, "euclidean"), (torch.float32, 32768, "offset", 16.0, "euclidean"),
+    (torch.float32, 16384, "offset", 0.985, "cosine")])
+def test_select_no_slower_than_the_serial_walk(gpu, dtype, N, kind, tau, metric):
+    """Keys that the banded walk is not for (few or no keys kept, fp32 keys close together against
+    their norms) take it no longer than the serial walk, which the same keys take when their rows
+    are not 16-byte aligned.  They once took up to four times as long."""
+    from deltaattention_amd import ops, synth
+    H, D = 8, 128
+    if kind == "ar":
+        k = synth.make_layer_inputs(1, H, H, N, D, seed=37)[1]
+    else:
+        gen = torch.Generator().manual_seed(41)
+        k = (torch.randn((1, H, N, D), generator=gen) if kind == "offset" else 0.0) + \
+            8.0 * torch.randn((1, H, 1, D), generator=gen)
+        k = k.expand(1, H, N, D)
+    k = k.to(dtype).to(gpu).contiguous()
+    wide = torch.zeros((1, H, N, D + 2), dtype=dtype, device=gpu)
+    wide[..., :D] = k
+    odd = wide[..., :D]
+    announce(f"select against the serial walk {dtype} N={N} {kind} tau={tau} {metric}")
+    keep, counts = ops.select(k, tau, 512, 0, metric)
+    bufs = keep, counts
+
+    def best_us(keys):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(10):
+                ops.select(keys, tau, 512, 0, metric, *bufs)
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = float("inf")
+        for _ in range(5):
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            best = min(best, 100.0 * a.elapsed_time(b))
+        return best
+    want = [t.clone() for t in ops.select(odd, tau, 512, 0, metric)]
+    assert torch.equal(keep, want[0]) and torch.equal(counts, want[1])
+    band, walk = best_us(k), best_us(odd)
+    print(f"{band:.1f} us, serial walk {walk:.1f}", flush=True)
+    assert band <= 1.2 * walk
