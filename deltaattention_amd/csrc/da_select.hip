@@ -604,7 +604,7 @@ void select_band_kernel(
   const int seg = blockDim.x;  // rows a segment: 64 a wave
   // the wave that joins the blocks and walks: another SIMD's for each of a CU's workgroups, in
   // whatever order it gets them
-  const int lead = (int)((blockIdx.x >> 3) + (blockIdx.x >> 8)) % min(seg / 64, 4);
+  const int lead = (int)((blockIdx.x >> 3) + (blockIdx.x >> 8)) & (seg >= 256 ? 3 : seg >= 128 ? 1 : 0);
   // ---- the walk of the rows from r on, two a step: both against the anchor, one a half, and
   // the second against the first (of two steps at once), which does not wait for the anchor.
   // Ends at the first anchor at or past `stop`, which it returns; the kept rows before go into
@@ -822,7 +822,7 @@ void select_band_kernel(
           }
           // ---- the anchors whose rows so far hold none: tile after tile, until all have one ----
           uint64_t want = __ballot(mine && (K | U) == 0 && tb + window_end() < e);
-          if (hard || want == 0) break;
+          if (__builtin_expect(hard || want == 0, 1)) break;
           s_ku[64 * wid + lane] = u32x4{(uint32_t)K, (uint32_t)(K >> 32), (uint32_t)U, (uint32_t)(U >> 32)};
 #pragma unroll 1
           for (int half = 0; half < 2; ++half) {
@@ -893,7 +893,7 @@ void select_band_kernel(
                                 (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(path[1]) << 32;
             bits |= on;
             count += __builtin_popcountll(on);
-            if (to < 0) {
+            if (__builtin_expect(to < 0, 0)) {
               // on from the anchor it stops at, past the blocks that were left to the walk
               const int pa = 64 * i + (-1 - to);
               int j = i + 1;
@@ -904,7 +904,7 @@ void select_band_kernel(
               p = 64 * i + to;
             }
           }
-          if (lane == 0) s_bits[i] |= bits;
+          if (lane == 0) atomicOr((unsigned long long*)&s_bits[i], (unsigned long long)bits);  // (no wait for a read)
         }
         if (lane == 0) s_cur = sb + p;
       }
