@@ -6,10 +6,10 @@
 // (deltaFlashAttention.py:9-357) with their wrappers (modeling_llama.py:306-451).
 //
 // Work decomposition.  A workgroup is 4 waves; each wave owns 64 query rows of one query
-// head.  The 4 waves always read the same KV head: with a GQA group of 4 they are 4 query
-// heads of the group on the same 64 rows, so every K/V tile staged in LDS serves 4 heads
-// (repeat_kv is never materialised).  With smaller groups the waves split 128 or 256 rows
-// instead.
+// head, or 32 where the grid is small (launch_attn_rows).  The 4 waves always read the same KV
+// head: with a GQA group of 4 they are 4 query heads of the group on the same 64 (32) rows, so
+// every K/V tile staged in LDS serves 4 heads (repeat_kv is never materialised).  With smaller
+// groups the waves split 128 or 256 (64 or 128) rows instead.
 //
 // Logical schedule (deltaFlashAttention.py:58-113).  Phase 1 takes packed blocks of
 // 128 anchors while their maximum timestamp is < start_m - W; Phase 2 covers dense
@@ -53,8 +53,6 @@ struct AttnArgs {
   const uint16_t* v;
   const uint16_t* kp;
   const uint16_t* vp;
-  const int32_t* ts;
-  const void* cnt;
   uint16_t* out;
   int64_t sq_b, sq_h, sq_n;
   int64_t sk_b, sk_h, sk_n;
@@ -62,8 +60,6 @@ struct AttnArgs {
   int64_t skp_b, skp_h, skp_n;
   int64_t svp_b, svp_h, svp_n;
   int64_t so_b, so_h, so_n;
-  int64_t sts_b, sts_h;
-  int64_t scnt_b, scnt_h;
   int B, Hq, Hkv, G, Nq, Nk;
   SeqMap seq;  // ragged batch (varlen): every sequence has Nq = Nk = seq.len(b)
   int D;  // head dimension: a multiple of 8, at most 128 (dims D..127 are zero-filled)
@@ -71,8 +67,6 @@ struct AttnArgs {
   const int32_t* P_dev;  // P on the device ([B], one per sequence, for a ragged batch)
   int window;
   float scale_log2;  // softmax scale * log2(e)
-  int no_count;
-  int cnt_is_float;
   int causal;
   const int32_t* sched;  // [B*Hkv][2][nblk_cap]: block maxima, prefix maxima
   int nblk_cap;
@@ -145,16 +139,14 @@ __device__ __forceinline__ const void* uniform_ptr(const void* p) {
   return (const void*)(((uint64_t)hi << 32) | lo);
 }
 
-// Workgroup barrier after the wave's own LDS reads and writes are done, leaving
-// loads to LDS (buffer_load ... lds) in flight.  A fence for LDS would wait for those
-// too (vmcnt(0)): the loads issued in this window are only read after the next
-// barrier, and their wait is explicit.  The asm is a compiler memory barrier.
-__device__ __forceinline__ void barrier_keep_loads() {
+// Workgroup barrier after the wave's own LDS reads and writes.  Its loads to LDS
+// (buffer_load ... lds) have their own wait, vmcnt(0), just before.  The asm is a compiler
+// memory barrier.
+__device__ __forceinline__ void window_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef short i16x8 __attribute__((ext_vector_type(8)));
 
 // LDS byte address of a pointer into the kernel's LDS.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
@@ -188,12 +180,6 @@ __device__ __forceinline__ void lgkm_wait(u32x4& a, u32x4& b) {
 template <int N>
 __device__ __forceinline__ void lgkm_wait(u32x4& a) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(a) : "i"(N));
-}
-// An unspecified value that costs no instruction: for a register array on a path where
-// it is dead, so that it is not live around the loop.
-template <typename T>
-__device__ __forceinline__ void undefined(T& x) {
-  asm volatile("" : "=v"(x));
 }
 template <typename F, int... I>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
@@ -431,9 +417,8 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   // steps of four: lane l writes 16 bytes at 1 KiB (2 w + j) + 16 l, i.e. row 8 w + 4 j + l / 16
   // at position l % 16, so it fetches the source chunk that the swizzled layout keeps there.  The buffer
   // resource covers exactly the tile's valid keys: rows past the end, and 8-dim chunks
-  // at or beyond the head dimension, arrive as zeros.  Each wave issues the same loads
-  // in every window, so the s_waitcnt vmcnt(n) at the end of a window, n = the loads of
-  // this window, waits exactly for those of the window before. ----
+  // at or beyond the head dimension, arrive as zeros.  A window's loads go out after its
+  // barrier, and all are waited for (vmcnt(0)) before the next one. ----
   const int wid_s = __builtin_amdgcn_readfirstlane(wid);
   const char* kb1 = (const char*)uniform_ptr(kp_base);
   const char* kb2 = (const char*)uniform_ptr(k_base);
@@ -738,7 +723,7 @@ __device__ __forceinline__ void attn_w64_item(const AttnArgs& a, const int unit,
   // window w - 1 (K of w + 1, V of w) are done: K of w + 2 and V of w + 1 take their stages.
   auto turn = [&](const int w) {
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-    barrier_keep_loads();
+    window_barrier();
     if (w < T) dma_issue(w + 2, w + 1, stA, stB);
   };
   auto swap_stages = [&]() {
@@ -1552,16 +1537,11 @@ static int hybrid_impl(const char* who, AttnArgs& a, const void* k_packed, const
   if (!workspace || workspace_bytes < need)
     return set_error(DA_ERR_WORKSPACE, "%s: workspace of %lld bytes required", who, (long long)need);
   a.kp = (const uint16_t*)k_packed; a.vp = (const uint16_t*)v_packed;
-  a.ts = timestamps; a.cnt = counts;
   a.skp_b = strides[DA_STRIDE_KP]; a.skp_h = strides[DA_STRIDE_KP + 1]; a.skp_n = strides[DA_STRIDE_KP + 2];
   a.svp_b = strides[DA_STRIDE_VP]; a.svp_h = strides[DA_STRIDE_VP + 1]; a.svp_n = strides[DA_STRIDE_VP + 2];
-  a.sts_b = strides[DA_STRIDE_TS]; a.sts_h = strides[DA_STRIDE_TS + 1];
-  a.scnt_b = strides[DA_STRIDE_CNT]; a.scnt_h = strides[DA_STRIDE_CNT + 1];
   a.P_host = (int)P_bound;
   a.P_dev = num_packed_dev;
   a.window = (int)window;
-  a.no_count = no_count ? 1 : 0;
-  a.cnt_is_float = counts_dtype == DA_F32;
   a.causal = 1;
   const HybridWs wl = hybrid_ws(B, Hkv, P_bound);
   char* ws = (char*)workspace;
@@ -1574,10 +1554,10 @@ static int hybrid_impl(const char* who, AttnArgs& a, const void* k_packed, const
   SchedPrep prep = {};
   if (variant != DA_VARIANT_SANITY) {
     prep.cnt = counts;
-    prep.scnt_b = a.scnt_b;
-    prep.scnt_h = a.scnt_h;
-    prep.cnt_is_float = a.cnt_is_float;
-    prep.no_count = a.no_count;
+    prep.scnt_b = strides[DA_STRIDE_CNT];
+    prep.scnt_h = strides[DA_STRIDE_CNT + 1];
+    prep.cnt_is_float = counts_dtype == DA_F32;
+    prep.no_count = no_count ? 1 : 0;
     prep.scale_log2 = a.scale_log2;
     prep.wts = (float*)(ws + wl.w_off);
     prep.tsw = variant == DA_VARIANT_PURE_PHASE1 ? (int32_t*)(ws + wl.ts_off) : nullptr;
@@ -1588,7 +1568,7 @@ static int hybrid_impl(const char* who, AttnArgs& a, const void* k_packed, const
   // the 16-bit kernel's persistent grid takes its items from 8 counters in the workspace
   a.queue = dtype != DA_F32 ? (int*)(ws + wl.queue_off) : nullptr;
   hipLaunchKernelGGL(hybrid_schedule_kernel, dim3((unsigned)(B * Hkv), 1 + prep_chunks), dim3(kSchedThreads), 0, st,
-                     timestamps, a.sts_b, a.sts_h, (int)Hkv, (int)P_bound, num_packed_dev, (int)Nk, a.seq,
+                     timestamps, strides[DA_STRIDE_TS], strides[DA_STRIDE_TS + 1], (int)Hkv, (int)P_bound, num_packed_dev, (int)Nk, a.seq,
                      a.nblk_cap, (int32_t*)ws, prep, a.queue);
   if (int rc = check_launch("hybrid prefill (schedule)")) return rc;
   const int kv = variant == DA_VARIANT_HYBRID ? kHybrid : (variant == DA_VARIANT_SANITY ? kSanity : kPure);
