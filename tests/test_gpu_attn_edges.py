@@ -43,9 +43,11 @@ def test_groups_and_row_edges(gpu, variant, B, Hq, Hkv, N, D, W, chunk):
 
 @pytest.mark.parametrize("Hq,Hkv,N,causal", [
     (1, 1, 1, True), (7, 7, 63, True), (2, 2, 256, False), (6, 3, 129, True), (32, 8, 1056, True),
-    (16, 16, 513, True), (40, 8, 300, False), (64, 16, 600, True)])
+    (16, 16, 513, True), (40, 8, 300, False), (64, 16, 600, True), (32, 8, 2048, False), (32, 8, 2080, False),
+    (300, 300, 100, False)])
 def test_dense_small_grids(gpu, Hq, Hkv, N, causal):
-    """Grids of less than one, between one and two, and more workgroups than run at once."""
+    """Grids of less than one, between one and two, and more workgroups than run at once; unmasked
+    ones on both sides of one 64-row item a CU and with half an item past the rows."""
     from deltaattention_amd import ops, synth
     q, k, v = synth.make_layer_inputs(1, Hq, Hkv, N, 128, seed=N)
     announce(f"dense Hq={Hq} Hkv={Hkv} N={N} causal={causal}")
@@ -79,12 +81,17 @@ def test_pure_phase1_unsorted_timestamps(gpu):
     (6, 3, 129, 128, 0, torch.bfloat16), (8, 1, 65, 128, 64, torch.float16), (12, 3, 193, 72, 64, torch.bfloat16),
     (8, 2, 1400, 128, 128, torch.bfloat16)])
 def test_32_row_waves_match_64_row_ones(gpu, variant, Hq, Hkv, N, D, W, dtype):
-    """A grid of at most one workgroup a CU takes 32 rows a wave instead of 64.  Every row's sums
-    are the same: a batch of copies, which fills the chip, repeats the one sequence's output
-    bit for bit."""
+    """A grid of at most two 64-row items a CU takes 32 rows a wave instead of 64.  Every row's
+    sums are the same: a batch of copies beyond that line repeats the one sequence's output bit
+    for bit."""
     from deltaattention_amd import ops, synth
     q, k, v = synth.make_layer_inputs(1, Hq, Hkv, N, D, seed=N, dtype=dtype, device=str(gpu))
-    copies = 1 + 256 // Hkv  # more units than CUs, whatever the rows
+    G = Hq // Hkv
+    hpw = 4 if G % 4 == 0 else 2 if G % 2 == 0 else 1   # query heads a workgroup takes
+    items = Hkv * (G // hpw) * -(-N // (256 // hpw))    # of one sequence, 64 rows a wave
+    line = 2 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    copies = 1 + line // items
+    assert items <= line < copies * items
     qb, kb, vb = (x.repeat(copies, 1, 1, 1) for x in (q, k, v))
     announce(f"32- and 64-row waves {variant} Hq={Hq} Hkv={Hkv} N={N} D={D} W={W} {dtype}")
     if variant == "dense":
@@ -129,5 +136,5 @@ def test_more_queries_than_keys(gpu, variant, Hq, Hkv, Nq, Nk, P, W, dtype):
     some = np.isfinite(want)
     assert np.isfinite(out)[some].all()
     err = np.abs(out - want)[some]
-    bars = (2e-5, 2e-6) if dtype == torch.float32 else (2e-2, 1e-3)
+    bars = (1e-5, 1e-6) if dtype == torch.float32 else (2e-2, 1e-3)
     assert err.max() <= bars[0] and err.mean() <= bars[1], (err.max(), err.mean())

@@ -90,8 +90,8 @@ def test_select_bitexact_config1_shape(gpu):
 ])
 def test_select_chunk_shapes(gpu, H, N, chunk, tau, metric, arith):
     """Selection against the sequential oracle over chunk lengths from 1 to 10000 rows,
-    grids of 2 to 2295 chunks (one chunk per wave below 2048, two from there on) and
-    thresholds that keep one row per chunk or nearly every row."""
+    grids of 2 to 2295 chunks (the banded walk up to 512, one chunk per wave from there on, two
+    from 2048) and thresholds that keep one row per chunk or nearly every row."""
     from deltaattention_amd import ops, synth
     k = synth.make_layer_inputs(1, H, H, N, 128, seed=21, rope_base=500000.0)[1]
     announce(f"select H={H} N={N} chunk={chunk} tau={tau} {metric} {arith}")
@@ -137,13 +137,13 @@ def test_select_native_arith_bitexact(gpu, dtype, oracle_arith):
 
 
 @pytest.mark.parametrize("scale,tau", [(2e-3, 0.015), (40.0, 250.0)], ids=["subnormal-squares", "near-fp16-max"])
-@pytest.mark.parametrize("H", [4, 64], ids=["one-chunk-per-wave", "two-chunks-per-wave"])
+@pytest.mark.parametrize("H", [4, 64], ids=["banded", "two-chunks-per-wave"])
 def test_select_fp16_native_extremes(gpu, scale, tau, H):
     """fp16 keys in the keys' own arithmetic at the edges of the format, bit-exact against
     the oracle's fp16 rounding (pinned against torch, subnormals included): keys scaled
     so that the squared differences are fp16 subnormals (spacing 6e-8) with the threshold
     among them, and keys whose distances reach the fp16 maximum (65504, spacing 32; sums
-    past it are inf, kept) with tau^2 = 62500 just below it.  Both walk layouts."""
+    past it are inf, kept) with tau^2 = 62500 just below it."""
     from deltaattention_amd import ops, synth
     N = 16384 if H == 64 else 4096   # 64 heads x 32 chunks: the pair walk's 2048 chunks
     k = (synth.make_layer_inputs(1, H, H, N, 128, seed=29, rope_base=10000.0)[1].float() * scale).to(torch.float16)
