@@ -932,8 +932,8 @@ static int launch_select(const void* k, int dtype, int64_t B, int64_t Hkv, int64
   // The banded walk takes rows it can read 16 bytes at a time.  The line is one round of the chip:
   // two workgroups a CU, one for fp32 keys (their registers).  There its time is 0.2 to 0.65 of
   // the serial walk's with one key in two to eight kept and about the serial walk's with keys that
-  // it leaves to its own (0.8 to 1.05, the worst found 1.15: 512 chunks of bf16 keys, one in
-  // sixteen kept, 83 against 73 us).  A second round doubles the latter and gains little on the
+  // it leaves to its own (0.8 to 1.05, the worst found 1.16: 512 chunks of bf16 keys, one in
+  // sixteen kept, 84 against 73 us).  A second round doubles the latter and gains little on the
   // former: 1024 chunks 46 us at one key in two, 78 at one in eight, 103 and more from one in sixteen
   // on, against 74; a look at a chunk's first 64 rows before the rest costs 6 us and leaves 97 to
   // 165.  Below 128 rows a chunk is too short to gain (97 rows, 680 chunks: 19.5 against 17.1 us).
