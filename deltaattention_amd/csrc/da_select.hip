@@ -485,6 +485,8 @@ struct BandTile {
 // after (a guarded load would be waited for before the next one).
 template <int DT, bool FULL>
 __device__ __forceinline__ void band_load(BandTile<DT>& x, const typename SelKey<DT>::Elem* row, int D, int hl) {
+  // opaque: the chunks' limits are formed here, not held in 16 scalar registers over the loops
+  if constexpr (!FULL) asm("" : "+s"(D));
   if constexpr (DT == DA_F32) {
     // converted here: the norm is of the fp32 elements, the products of their bf16 roundings
     f32x4 lo[8], hi[8];
@@ -546,10 +548,10 @@ __device__ __forceinline__ float band_norm(const BandTile<DT>& x, int ql, int hl
   return n + swap_halves(n);
 }
 
-// FULL: D = 128 (rows at immediate offsets from one address; two workgroups a CU then fit
-// the registers of the Euclidean walk on 16-bit keys).
+// FULL: D = 128 (rows at immediate offsets from one address; the registers of 16-bit keys then
+// hold two workgroups a CU).
 template <bool COS, bool A16, int DT, bool FULL>
-__global__ __launch_bounds__(64 * kBandWaves) __attribute__((amdgpu_waves_per_eu(FULL && !COS && DT != DA_F32 ? 4 : 2)))
+__global__ __launch_bounds__(64 * kBandWaves) __attribute__((amdgpu_waves_per_eu(FULL && DT != DA_F32 ? 4 : 2)))
 void select_band_kernel(
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int H, int64_t N,
     int D_arg, int cs, int nc, float thr, BandBounds bounds, int32_t* __restrict__ keep,
@@ -930,16 +932,18 @@ static int launch_select(const void* k, int dtype, int64_t B, int64_t Hkv, int64
   const int64_t blocks = (total + 3) / 4;
   DA_REQUIRE(blocks < (1ll << 31), "%s: too many chunks", who);
   // The banded walk takes rows it can read 16 bytes at a time.  The line is one round of the chip:
-  // two workgroups a CU, one for fp32 keys (their registers).  There its time is 0.2 to 0.65 of
-  // the serial walk's with one key in two to eight kept and about the serial walk's with keys that
-  // it leaves to its own (0.8 to 1.05, the worst found 1.16: 512 chunks of bf16 keys, one in
-  // sixteen kept, 84 against 73 us).  A second round doubles the latter and gains little on the
-  // former: 1024 chunks 46 us at one key in two, 78 at one in eight, 103 and more from one in sixteen
-  // on, against 74; a look at a chunk's first 64 rows before the rest costs 6 us and leaves 97 to
-  // 165.  Below 128 rows a chunk is too short to gain (97 rows, 680 chunks: 19.5 against 17.1 us).
+  // two workgroups a CU, one for fp32 keys or other than 128 dims (their registers; fp32 keys of
+  // other than 128 dims half a round, 64 chunks 59 against 60 us but 256 77 / 63 with few kept).
+  // There its time is 0.2 to 0.65 of the serial walk's with one key in two to eight kept and about
+  // the serial walk's with keys that it leaves to its own (0.8 to 1.05, the worst found 1.16: 512
+  // chunks of bf16 keys, one in sixteen kept, 84 against 73 us).  A second round doubles the latter
+  // and gains little on the former: 1024 chunks 46 us at one key in two, 78 at one in eight, 103 and
+  // more from one in sixteen on, against 74; a look at a chunk's first 64 rows before the rest costs
+  // 6 us and leaves 97 to 165.  Below 128 rows a chunk is too short to gain (97 rows, 680 chunks:
+  // 19.5 against 17.1 us).
   const int per16 = dtype == DA_F32 ? 4 : 8;
   const int64_t rows = seq.cu && divide_to > 0 ? (N + divide_to - 1) / divide_to : std::min(chunk_size, N);
-  const int64_t band_max = dtype == DA_F32 ? 256 : 512;
+  const int64_t band_max = (dtype == DA_F32 ? 256 : 512) / (D == 128 ? 1 : 2);
   if (rows >= kBandMinRows && total <= band_max && (D & 7) == 0 && ((sk_b | sk_h | sk_n) % per16) == 0 &&
       ((uintptr_t)k & 15) == 0 && std::isfinite(threshold)) {
     const BandBounds bounds = band_bounds(use_cosine, a16, dtype, threshold);

@@ -623,14 +623,15 @@ def test_select_fp16_native_extremes_serial(gpu, scale, tau):
     (torch.bfloat16, 65536, "ar", 15.9, "euclidean"), (torch.bfloat16, 32768, "constant", 0.5, "euclidean"),
     (torch.bfloat16, 32768, "ar", -2.0, "cosine"), (torch.float16, 32768, "ar", 1e6, "euclidean"),
     (torch.float32, 16384, "offset", 16.0, "euclidean"), (torch.float32, 32768, "offset", 16.0, "euclidean"),
-    (torch.float32, 16384, "offset", 0.985, "cosine")])
+    (torch.float32, 16384, "offset", 0.985, "cosine"), (torch.bfloat16, 16384, "ar 64 dims", 1e6, "euclidean"),
+    (torch.bfloat16, 32768, "ar 64 dims", 11.2, "euclidean"), (torch.float32, 8192, "ar 64 dims", 1e6, "euclidean")])
 def test_select_no_slower_than_the_serial_walk(gpu, dtype, N, kind, tau, metric):
     """Keys that the banded walk is not for (few or no keys kept, fp32 keys close together against
     their norms) take it no longer than the serial walk, which the same keys take when their rows
     are not 16-byte aligned.  They once took up to four times as long."""
     from deltaattention_amd import ops, synth
-    H, D = 8, 128
-    if kind == "ar":
+    H, D = 8, 64 if kind.endswith("64 dims") else 128
+    if kind.startswith("ar"):
         k = synth.make_layer_inputs(1, H, H, N, D, seed=37)[1]
     else:
         gen = torch.Generator().manual_seed(41)
