@@ -253,8 +253,8 @@ constexpr float kLazySum = 16.0f * 256.0f;
 // 1.97 against 2.04 ms, 131072 27.9 / 28.7; ragged batches 4.5 / 4.7 ms).  It reads each tile
 // twice as often from L2, which costs up to 0.3 % where neither matters (dense 32768).  Groups
 // that are not a multiple of 4 ran a 32-row kernel that staged tiles through registers: 8000
-// tokens x 32 heads, keys repeated to the query heads, 286 against 319 us (236 with the lazy
-// maximum below).
+// tokens x 32 heads, keys repeated to the query heads, 264 against 319 us (286 with the queues,
+// 236 with them and the lazy maximum below).
 // ====================================================================================
 constexpr int kWTK = 32;                         // keys per tile
 constexpr int kWKBytes = kWTK * kD * 2;          // 8 KiB
